@@ -277,22 +277,13 @@ int library_workspace(int dev, hipStream_t stream, size_t bytes, void** out) {
 // can see bounds every sequence's count.
 struct SplitPlan {
   int max_splits;
-  int runs_cap;  // per-query split: runs of the longest sequence (0: whole-call split)
+  int query_chunks;  // per-query split: chunks of the longest query (0: whole-call split)
 };
 
 SplitPlan plan_splits(int64_t max_tokens) { return {jacq::split_count(max_tokens), 0}; }
 
-// Per-query split plan: a query of up to max_tokens tokens is cut into at
-// most this many runs (the kernel's stream_waves of its units).
-// A query of at most max_tokens tokens has T <= ceil(max_tokens / 32) tiles,
-// at most R / 32 + 1 of them fp16 residual tiles, so its units (quantised
-// groups + 3 per residual tile = T + 2 residual tiles) are bounded by
-// T + 2 (R / 32 + 1) per kv head, whatever its length.
-SplitPlan plan_splits_per_query(const KiviGeo& g, int64_t max_tokens, int waves) {
-  const int64_t tiles = std::max<int64_t>(1, (max_tokens + jacq::kGroup - 1) / jacq::kGroup);
-  const int64_t units = (int64_t)g.nkv * (tiles + 2 * (g.residual / jacq::kGroup + 1));
-  const int64_t runs = std::min<int64_t>(waves, std::max<int64_t>(1, (units + 3) / 4));
-  return {jacq::split_count(max_tokens), (int)runs};
+SplitPlan plan_splits_per_query(const KiviGeo& g, int64_t max_tokens, int cus) {
+  return {jacq::split_count(max_tokens), jacq::plan_chunks(g, 1, max_tokens, true, cus).per_query};
 }
 
 // JACQ_KIVI_DECODE=simple selects the VALU decode kernel (a cross-check of
@@ -306,14 +297,14 @@ bool use_simple_decode() {
 }
 
 // Partial-result slots: VALU kernel -- one per (sequence, kv head, split);
-// matrix-core kernel -- one per (sequence, kv head) plus one per wavefront
-// (a wavefront's run cuts at most one extra piece off the stream).
-// Per-query split (the v1 symbols): one per (query, kv head) plus one per
-// run of each query, at most runs_cap (the runs of the longest sequence).
+// matrix-core kernels -- one per (sequence, kv head) plus one per wavefront
+// (a wavefront's run cuts at most one extra piece off the stream; the chunk
+// kernel makes no more chunks than workgroups are resident).
+// Per-query split (the v1 symbols): one per chunk of each query.
 size_t partial_slots(const KiviGeo& g, int batch, const SplitPlan& sp, int waves) {
   if (use_simple_decode())
     return sp.max_splits <= 1 ? 0 : (size_t)batch * g.nkv * sp.max_splits;
-  if (sp.runs_cap > 0) return (size_t)batch * ((size_t)g.nkv + (size_t)sp.runs_cap);
+  if (sp.query_chunks > 0) return (size_t)batch * (size_t)sp.query_chunks;
   return (size_t)batch * g.nkv + (size_t)waves;
 }
 
@@ -338,7 +329,7 @@ void fill_ws(jacq::DecodeArgs& a, const KiviGeo& g, int batch, const SplitPlan& 
   a.max_splits = sp.max_splits;
   a.batch = batch;
   a.waves = waves;
-  a.per_query = sp.runs_cap > 0;
+  a.per_query = sp.query_chunks > 0;
   const size_t slots = partial_slots(g, batch, sp, waves) * g.gqa;
   a.ws_poison = (uint64_t*)ws;
   a.ws_ml = ws ? (float*)((uint8_t*)ws + kWorkspaceHeader) : nullptr;
@@ -428,7 +419,7 @@ int run_decode(const jacq_kivi_geometry& x, const jacq_half_t* Q, const int32_t*
   // the writer wavefronts are stream wavefronts: never more than the grid holds
   const int nw = step ? std::min(step_writer_waves(g, batch), waves) : 0;
   const SplitPlan sp =
-      per_query ? plan_splits_per_query(g, max_tokens, waves) : plan_splits(max_tokens);
+      per_query ? plan_splits_per_query(g, max_tokens, ds.cus) : plan_splits(max_tokens);
   const size_t need = workspace_bytes(g, batch, sp, waves) + (step ? step_flag_bytes(g, batch) : 0);
   if (need > 0) {
     if (ws == nullptr) {
@@ -465,7 +456,16 @@ int run_decode(const jacq_kivi_geometry& x, const jacq_half_t* Q, const int32_t*
   a.retained_pages = retained_pages;
   a.status = ds.status_dev;
   fill_ws(a, g, batch, sp, waves, need > 0 ? ws : nullptr);
+  if (!use_simple_decode()) {
+    const jacq::ChunkPlan cp = jacq::plan_chunks(g, batch, max_tokens, per_query, ds.cus);
+    a.chunk_waves = cp.waves;
+    a.chunk_grid = cp.grid;
+    a.chunk_slots = cp.slots;
+    a.chunk_units = cp.units;
+    a.chunk_whole = cp.whole;
+  }
   if (step) {
+    a.fused = 1;
     a.wr = *step;
     a.writer_waves = nw;
     // the writer flags follow the split-K workspace
@@ -539,8 +539,9 @@ int v1_decode(const jacq_kivi_geometry& x, const jacq_half_t* Q, const int32_t* 
   void* region = nullptr;
   if (int e = v1_region(dev, stream, &region)) return e;
   const KiviGeo g = make_geo(x);
-  const int waves = jacq::decode_stream_waves(g, device_state(dev).cus);
-  const SplitPlan sp = plan_splits_per_query(g, max_seq_len(x), waves);
+  const int cus = device_state(dev).cus;
+  const int waves = jacq::decode_stream_waves(g, cus);
+  const SplitPlan sp = plan_splits_per_query(g, max_seq_len(x), cus);
   const size_t one = workspace_bytes(g, 1, sp, waves);
   const size_t per = one > kWorkspaceHeader ? one - kWorkspaceHeader : 0;
   const int chunk =

@@ -1,5 +1,9 @@
 // kivi_decode_mfma.hip -- paged int4-KIVI decode attention on CDNA4 matrix cores.
 //
+// Two decompositions share the tile loop (decode_tiles): the stream below, and
+// for calls of few segments, and the v1 symbols, chunks of segments folded within
+// workgroups (kivi_decode_chunk_kernel).
+//
 // Work decomposition ("stream" split-K).  Every (sequence, kv head) is a
 // stream of 32-token tiles (its quantised groups, then its fp16 residual
 // tokens); the streams of the whole batch are concatenated and cut into one
@@ -43,7 +47,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "kivi_kernels.h"
+#include "kivi_quant.h"
 
 namespace jacq {
 
@@ -430,10 +434,10 @@ struct PStash {
   __device__ explicit PStash(uint8_t* bytes) : base((float*)bytes) {}
   __device__ void put(const float (&p)[8]) const {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) base[64 * i + threadIdx.x] = p[i];
+    for (int i = 0; i < 8; ++i) base[64 * i + (threadIdx.x & 63)] = p[i];
   }
   __device__ float get(int i) const {
-    int o = threadIdx.x;
+    int o = threadIdx.x & 63;
     asm volatile("" : "+v"(o));
     return base[64 * i + o];
   }
@@ -784,20 +788,18 @@ __device__ inline int tile_at(int u, int nq) {
   return u <= nq ? u : nq + (u - nq + kResidualUnits - 1) / kResidualUnits;
 }
 
-__device__ inline int wave_sum_i(int v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// Inclusive sum over the wavefront's lanes, by data-parallel-primitive moves
+// (no LDS round trips: the plan of a call is on its critical path).
+__device__ inline int wave_incl_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1, within 16 lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2, 3
   return v;
 }
-
-__device__ inline int wave_incl_scan(int v, int lane) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(v, off, 64);
-    if (lane >= off) v += t;
-  }
-  return v;
-}
+__device__ inline int wave_sum_i(int v) { return __builtin_amdgcn_readlane(wave_incl_scan(v), 63); }
 
 // Total tiles of the concatenated streams (all sequences x kv heads).
 __device__ inline int64_t stream_units(const KiviGeo& g, const DecodeArgs& a, int lane) {
@@ -805,7 +807,7 @@ __device__ inline int64_t stream_units(const KiviGeo& g, const DecodeArgs& a, in
   for (int base = 0; base < a.batch; base += 64) {
     int U = 0;
     if (base + lane < a.batch) U = seq_units(g, a, base + lane);
-    tot += __builtin_amdgcn_readfirstlane(wave_sum_i(U));
+    tot += wave_sum_i(U);
   }
   return tot * g.nkv;
 }
@@ -814,14 +816,10 @@ __device__ inline int64_t stream_units(const KiviGeo& g, const DecodeArgs& a, in
 // kMinUnitsPerWave units each, so that small batches spread over enough
 // wavefronts to hide the per-group latency chain without cutting every
 // segment into pieces the merge must fold (4: TinyLlama 17.9 -> 15.6 us,
-// Qwen0.5B 19.6 -> 18.5 us against 8; 2 was slower at Qwen0.5B).  A whole
-// call's stream of fewer than kTinyStream units (TinyLlama's 72) takes 2 per
-// wavefront (0.9 us faster there; 1 was slower).  The per-query split keeps
-// 4: the host sizes its partial slots from that.
-constexpr int kMinUnitsPerWave = 4, kTinyStream = 256;
-__device__ inline int64_t stream_waves(int64_t units, int grid, bool whole_call = false) {
-  const int per = whole_call && units < kTinyStream ? 2 : kMinUnitsPerWave;
-  int64_t w = (units + per - 1) / per;
+// Qwen0.5B 19.6 -> 18.5 us against 8; 2 was slower at Qwen0.5B).
+constexpr int kMinUnitsPerWave = 4;
+__device__ inline int64_t stream_waves(int64_t units, int grid) {
+  int64_t w = (units + kMinUnitsPerWave - 1) / kMinUnitsPerWave;
   if (w < 1) w = 1;
   return w < grid ? w : grid;
 }
@@ -840,7 +838,7 @@ __device__ inline SeqSpan locate(const KiviGeo& g, const DecodeArgs& a, int64_t 
     const int bb = base + lane;
     int T = 0;
     if (bb < a.batch) T = seq_units(g, a, bb);
-    const int incl = wave_incl_scan(T, lane);
+    const int incl = wave_incl_scan(T);
     const uint64_t hit = __builtin_amdgcn_ballot_w64(bb < a.batch && run + (int64_t)g.nkv * incl > x);
     if (hit) {
       const int f = __builtin_ctzll(hit);
@@ -924,59 +922,6 @@ __device__ inline ResTile<HD> load_res(const DecodeArgs& a, const KiviGeo& g, in
   return rt;
 }
 
-// ---- per-query split (the v1 symbols) ----
-//
-// Each query's streams (NKV x its units) are cut into stream_waves(its units)
-// equal runs by its own length alone, exactly as a call with that query alone
-// cuts them, whatever the other queries of the call are: every query decodes
-// to the same bits in a batched call as in a single one (variants.rs:1211-1213
-// expects the batched kernel to match the single-token one bit for bit).  The
-// runs of all queries are numbered query by query; the stream wavefronts take
-// them in turn.
-struct RunLoc {
-  int q;       // query, or -1 past the last run
-  int units;   // units per kv head of the query
-  int runs;    // runs of the query
-  int64_t r0;  // global index of the query's first run
-};
-
-__device__ inline int query_runs(const KiviGeo& g, const DecodeArgs& a, int units) {
-  return (int)stream_waves((int64_t)g.nkv * units, a.waves);
-}
-
-__device__ inline RunLoc locate_run(const KiviGeo& g, const DecodeArgs& a, int64_t r, int lane) {
-  int64_t acc = 0;
-  for (int base = 0; base < a.batch; base += 64) {
-    const int bb = base + lane;
-    int U = 0, R = 0;
-    if (bb < a.batch) {
-      U = seq_units(g, a, bb);
-      R = query_runs(g, a, U);
-    }
-    const int incl = wave_incl_scan(R, lane);
-    const uint64_t hit = __builtin_amdgcn_ballot_w64(bb < a.batch && acc + incl > r);
-    if (hit) {
-      const int f = __builtin_ctzll(hit);
-      const int Rf = __builtin_amdgcn_readlane(R, f);
-      return {base + f, __builtin_amdgcn_readlane(U, f), Rf,
-              acc + __builtin_amdgcn_readlane(incl, f) - Rf};
-    }
-    acc += __builtin_amdgcn_readlane(incl, 63);
-  }
-  return {-1, 0, 0, acc};
-}
-
-// Global index of query b's first run.
-__device__ inline int64_t query_run_start(const KiviGeo& g, const DecodeArgs& a, int b, int lane) {
-  int64_t run = 0;
-  for (int base = 0; base < b; base += 64) {
-    const int bb = base + lane;
-    const int R = bb < b ? query_runs(g, a, seq_units(g, a, bb)) : 0;
-    run += __builtin_amdgcn_readfirstlane(wave_sum_i(R));
-  }
-  return run;
-}
-
 // The step's sequence b ages a group out: its old-token count grows.
 __device__ inline bool step_ages(const KiviGeo& g, int len_after) {
   return len_after >= 1 &&
@@ -1025,7 +970,7 @@ __device__ inline int64_t seq_start(const KiviGeo& g, const DecodeArgs& a, int b
   for (int base = 0; base < b; base += 64) {
     const int bb = base + lane;
     const int U = bb < b ? seq_units(g, a, bb) : 0;
-    run += __builtin_amdgcn_readfirstlane(wave_sum_i(U));
+    run += wave_sum_i(U);
   }
   return run * g.nkv;
 }
@@ -1114,17 +1059,16 @@ __device__ inline void write_stamp(const DecodeArgs& a, uint64_t t0, uint64_t in
 // likewise, O = acc / max(L, 1e-30), in the log2 domain of the decode loop.
 // The pieces of a segment are recomputed from the same split the stream
 // wavefronts used; a segment with a single non-empty piece was written whole.
-template <int HD, bool PACK, bool PQ, bool FUSED>
+template <int HD, bool PACK, bool FUSED>
 __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const KiviGeo& g,
                                                                        const DecodeArgs& a,
                                                                        int lane) {
   constexpr int K = (PACK ? 8 : 16) * HD / 256;  // float4 outputs per lane: G * HD <= 256 K
   constexpr int U = K <= 2 ? 8 : K > 4 ? 1 : 2;  // partials whose loads are in flight together
   const int G = g.gqa, NKV = g.nkv, n4 = G * HD / 4;
-  // the whole call's stream (per-query split: each segment's own query, below)
-  const int64_t TT = PQ ? 0 : stream_units(g, a, lane);
-  const int64_t W = PQ ? 0 : stream_waves(TT, a.waves, true);
-  const int64_t nw = FUSED ? a.writer_waves : 0;  // writer runs (PQ: none)
+  const int64_t TT = stream_units(g, a, lane);
+  const int64_t W = stream_waves(TT, a.waves);
+  const int64_t nw = FUSED ? a.writer_waves : 0;  // writer runs
   const int nseg = a.batch * NKV;
   const uint64_t epoch = a.epoch + a.merge_skew, t_start = __builtin_amdgcn_s_memrealtime();
   // wave-uniform: the wait ran out.  A merge of an earlier launch on this
@@ -1150,23 +1094,13 @@ __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const K
     const int T = seq_tiles(g, a, b, &ov, &n);
     const int nq = ov / kGroup;
     const int units = nq + kResidualUnits * (T - nq);
-    // the stream the segment's runs cut (sq units in wq runs), the segment's
-    // first unit in it, and the global index of that stream's first run
-    int64_t sq = TT, wq = W, S0, roff = 0;
-    if constexpr (PQ) {
-      sq = (int64_t)NKV * units;
-      wq = stream_waves(sq, a.waves);
-      S0 = (int64_t)h * units;
-      roff = query_run_start(g, a, b, lane);
-    } else {
-      S0 = seq_start(g, a, b, lane) + (int64_t)h * units;
-    }
+    const int64_t S0 = seq_start(g, a, b, lane) + (int64_t)h * units;
     const int64_t S1 = S0 + units;
-    const int64_t w0 = wave_of(S0, sq, wq, nw), w1 = wave_of(S1 - 1, sq, wq, nw);
+    const int64_t w0 = wave_of(S0, TT, W, nw), w1 = wave_of(S1 - 1, TT, W, nw);
     // non-empty pieces: the runs that own at least one tile of the segment
     auto owns = [&](int64_t w) {
-      const int64_t x0 = max(run_begin(w, sq, wq, nw), S0),
-                    x1 = min(run_begin(w + 1, sq, wq, nw), S1);
+      const int64_t x0 = max(run_begin(w, TT, W, nw), S0),
+                    x1 = min(run_begin(w + 1, TT, W, nw), S1);
       return tile_at((int)(x0 - S0), nq) < tile_at((int)(x1 - S0), nq);
     };
     int pieces = 0;
@@ -1186,7 +1120,7 @@ __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const K
     for (int64_t wb = w0; wb <= w1 && !late; wb += 64) {
       const int64_t wl = wb + lane;
       const bool mine = wl <= w1 && owns(wl);
-      const uint64_t* flag = a.ws_flag + seg + roff + wl;
+      const uint64_t* flag = a.ws_flag + seg + wl;
       uint64_t todo = __builtin_amdgcn_ballot_w64(mine);
       // fold the partials in piece order (the result does not depend on
       // timing), each run of them as soon as its flags show this launch's
@@ -1221,7 +1155,7 @@ __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const K
           for (int u = 0; u < U; ++u) {
             slot[u] = -1;
             if (ready) {
-              slot[u] = seg + roff + wb + __builtin_ctzll(ready);
+              slot[u] = seg + wb + __builtin_ctzll(ready);
               ready &= ready - 1;
             }
           }
@@ -1251,7 +1185,7 @@ __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const K
           // read: clear the flags, so the next launch starts from zero even
           // when it carries the same epoch (a replayed graph does)
           if (consumed & bit)
-            __hip_atomic_store(a.ws_flag + seg + roff + wl, 0ull, __ATOMIC_RELAXED,
+            __hip_atomic_store(a.ws_flag + seg + wl, 0ull, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
           for (int u = 0; u < U; ++u) {
@@ -1322,156 +1256,6 @@ constexpr int step_flags() {
   return 2 * (HD / kGroup);
 }
 
-// One age-out item: channels [32 q, 32 q + 32) of K or V of (sequence b, kv
-// head h).  The slice is self-contained: K is quantised per channel (over the
-// group's 32 tokens) and V per (token, 32-channel group), so the slice's codes
-// and scales need only its own rows, and the slice's shift touches no other
-// item's bytes -- items need no ordering among themselves.
-template <int HD>
-__device__ __attribute__((always_inline)) inline void step_age_out(const KiviGeo& g,
-                                                                   const DecodeArgs& a, int b,
-                                                                   int h, bool is_v, int q,
-                                                                   int lane) {
-#pragma clang fp contract(off)
-  constexpr int HDP = HD / 2, HDG = HD / kGroup;
-  const AppendArgs& w = a.wr;
-  const int P = g.page, ppg = kGroup / P;
-  const int start = step_len(a, b) - 1;
-  const int old0 = split_old_tokens(start, g.residual), r0 = start - old0;  // r0 = R + 31
-  uint16_t* xs = (is_v ? w.v_scr : w.k_scr) + (int64_t)b * w.scr_stride + (int64_t)h * g.rs * HD +
-                 kGroup * q;
-  const uint16_t* nx =
-      (is_v ? w.new_v : w.new_k) + (int64_t)b * w.new_stride + (int64_t)h * HD + kGroup * q;
-  const int fp = (old0 / kGroup) * ppg;  // the group's first logical page
-  const bool table_ok = fp + ppg <= g.max_pages;
-  int p0 = -1, p1 = -1;
-  if (table_ok) {
-    const int32_t* bt = w.block_tables + (int64_t)b * w.bt_stride;
-    p0 = bt[fp];
-    p1 = ppg == 2 ? bt[fp + 1] : p0;
-  }
-  auto phys_ok = [&](int p) { return table_ok && p >= 0 && p < g.num_pages; };
-  if (!is_v) {
-    // K: lane = (channel pair pr of the slice's 16, token quarter tq): the
-    // pair's min / max over its 8 tokens, merged over the 4 quarters
-    const int pr = lane >> 2, tq = lane & 3, t0 = 8 * tq;
-    uint32_t x[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) x[t] = *(const uint32_t*)(xs + (t0 + t) * HD + 2 * pr);
-    float mn0 = h2f((uint16_t)x[0]), mx0 = mn0, mn1 = h2f((uint16_t)(x[0] >> 16)), mx1 = mn1;
-#pragma unroll
-    for (int t = 1; t < 8; ++t) {
-      const float v0 = h2f((uint16_t)x[t]), v1 = h2f((uint16_t)(x[t] >> 16));
-      mn0 = min_num(mn0, v0);
-      mx0 = max_num(mx0, v0);
-      mn1 = min_num(mn1, v1);
-      mx1 = max_num(mx1, v1);
-    }
-#pragma unroll
-    for (int off = 1; off < 4; off <<= 1) {
-      mn0 = min_num(mn0, __shfl_xor(mn0, off, 64));
-      mx0 = max_num(mx0, __shfl_xor(mx0, off, 64));
-      mn1 = min_num(mn1, __shfl_xor(mn1, off, 64));
-      mx1 = max_num(mx1, __shfl_xor(mx1, off, 64));
-    }
-    float s0 = (mx0 - mn0) / 15.0f, s1 = (mx1 - mn1) / 15.0f;
-    if (!(s0 > 0.0f)) s0 = 1.0f;
-    if (!(s1 > 0.0f)) s1 = 1.0f;
-    const int d0 = kGroup * q + 2 * pr;  // channel of the pair's low nibble
-    if (tq == 0) {
-      const uint32_t sc = (uint32_t)f2h(s0) | ((uint32_t)f2h(s1) << 16);
-      const uint32_t zr = (uint32_t)f2h(mn0) | ((uint32_t)f2h(mn1) << 16);
-      for (int pg = 0; pg < ppg; ++pg) {  // K scales live in every page of the group
-        const int phys = pg == 0 ? p0 : p1;
-        if (!phys_ok(phys)) continue;
-        const int64_t base = ((int64_t)phys * g.nkv + h) * HD + d0;
-        st_dev((uint32_t*)(w.k_scale + base), sc);
-        st_dev((uint32_t*)(w.k_zero + base), zr);
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int tok = t0 + t, phys = tok < P ? p0 : p1;
-      const int c0 = clamp_code((h2f((uint16_t)x[t]) - mn0) / s0);
-      const int c1 = clamp_code((h2f((uint16_t)(x[t] >> 16)) - mn1) / s1);
-      if (phys_ok(phys))
-        st_dev(w.k_code + (((int64_t)phys * g.nkv + h) * P + tok % P) * HDP + d0 / 2,
-               (uint8_t)((c0 & 0x0f) | ((c1 & 0x0f) << 4)));
-    }
-  } else {
-    // V: lane = (token t, half hf of the slice's 32 channels); min / max over
-    // 16 channels, merged with the other half
-    const int t = lane >> 1, hf = lane & 1;
-    const uint16_t* row = xs + t * HD + 16 * hf;
-    const u32x4 v0 = *(const u32x4*)row, v1 = *(const u32x4*)(row + 8);
-    auto ch = [&](int k) -> float {  // channel k of the lane's 16
-      const u32x4& v = k < 8 ? v0 : v1;
-      return h2f((uint16_t)(v[(k % 8) / 2] >> (16 * (k & 1))));
-    };
-    float mn = ch(0), mx = mn;
-#pragma unroll
-    for (int k = 1; k < 16; ++k) {
-      mn = min_num(mn, ch(k));
-      mx = max_num(mx, ch(k));
-    }
-    mn = min_num(mn, __shfl_xor(mn, 1, 64));
-    mx = max_num(mx, __shfl_xor(mx, 1, 64));
-    float sv = (mx - mn) / 15.0f;
-    if (!(sv > 0.0f)) sv = 1.0f;
-    u32x2 codes;
-#pragma unroll
-    for (int wd = 0; wd < 2; ++wd) {
-      uint32_t word = 0;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) word |= (uint32_t)clamp_code((ch(8 * wd + k) - mn) / sv) << (4 * k);
-      codes[wd] = word;
-    }
-    const int phys = t < P ? p0 : p1;
-    if (phys_ok(phys)) {
-      const int64_t tok = ((int64_t)phys * g.nkv + h) * P + t % P;
-      st_dev((uint64_t*)(w.v_code + tok * HDP + q * (kGroup / 2) + 8 * hf),
-             __builtin_bit_cast(uint64_t, codes));
-      if (hf == 0) {
-        st_dev(w.v_scale + tok * HDG + q, f2h(sv));
-        st_dev(w.v_zero + tok * HDG + q, f2h(mn));
-      }
-    }
-  }
-  // shift the slice: rows [0, R - 1) <- rows [32, R + 31), four 16-byte
-  // pieces per row, in chunks of 8 pieces per lane.  Within a chunk store k
-  // writes rows that no later load of any chunk reads (sources lie 32 rows
-  // above), and the quantisation above read rows 0..31 first.
-  const int units = (g.residual - 1) * 4;
-  for (int u0 = 0; u0 < units; u0 += 64 * 8) {
-    u32x4 buf[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int u = min(u0 + lane + 64 * k, units - 1);
-      buf[k] = *(const u32x4*)(xs + (int64_t)(u / 4 + kGroup) * HD + 8 * (u % 4));
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int u = u0 + lane + 64 * k;
-      if (u < units)
-        st_agent4((float*)(xs + (int64_t)(u / 4) * HD + 8 * (u % 4)),
-                  __builtin_bit_cast(floatx4, buf[k]));
-    }
-  }
-  // the new token's slice: row R - 1 (live) and row r0 (the reference's stale copy)
-  if (lane < 8) {
-    const int row = lane < 4 ? g.residual - 1 : r0, piece = lane % 4;
-    st_agent4((float*)(xs + (int64_t)row * HD + 8 * piece),
-              __builtin_bit_cast(floatx4, *(const u32x4*)(nx + 8 * piece)));
-  }
-  // every store above is device-scope (the readers' loads are too): complete
-  // before the flag
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  if (lane == 0)
-    __hip_atomic_store(a.ws_wflag + step_flags<HD>() * ((int64_t)b * g.nkv + h) +
-                           (is_v ? HDG : 0) + q,
-                       a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Writer wavefront wi of a.writer_waves: first the age-out items (sequence
 // rank among the aging ones, kv head, K | V) in turn, then the plain appends
 // of the other (sequence, kv head) pairs.
@@ -1481,27 +1265,44 @@ __device__ __attribute__((always_inline)) inline uint64_t step_writer(const Kivi
   const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
   uint64_t tf = t0;  // profiling: the end of its last age-out item
   const int NW = a.writer_waves, NKV = g.nkv;
-  int rank0 = 0;  // aging sequences before this 64-sequence window
+  // An item's flag is stored once its (device-scope; the readers' loads are too)
+  // stores are complete: when the next item's loads have landed, so that an
+  // item's stores and the next one's loads share a memory round (64 sequences aging
+  // at once at 14B).
+  int done = -1;
+  auto publish = [&] {
+    if (done >= 0 && lane == 0)
+      __hip_atomic_store(a.ws_wflag + done, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    done = -1;
+  };
+  // this wavefront's items are wi, wi + NW, ... of (aging sequence, kv head, flag)
+  constexpr int F = step_flags<HD>();  // items per (sequence, kv head)
+  const int per = F * NKV;
+  int item = wi, first = 0;  // first: items of the windows before this one
   for (int base = 0; base < a.batch; base += 64) {
     const int bb = base + lane;
-    const bool ag = bb < a.batch && step_ages(g, step_len(a, bb));
-    uint64_t m = __builtin_amdgcn_ballot_w64(ag);
-    int rank = rank0;
-    while (m) {
-      const int b = base + __builtin_ctzll(m);
-      m &= m - 1;
-      constexpr int F = step_flags<HD>();  // items per (sequence, kv head)
-      for (int k = 0; k < F * NKV; ++k) {
-        const int item = rank * F * NKV + k;
-        if (item % NW == wi) {
-          const int hh = k / F, f = k % F;
-          step_age_out<HD>(g, a, b, hh, f >= F / 2, f % (F / 2), lane);
-          tf = __builtin_amdgcn_s_memrealtime();
-        }
-      }
-      ++rank;
+    uint64_t m = __builtin_amdgcn_ballot_w64(bb < a.batch && step_ages(g, step_len(a, bb)));
+    const int end = first + per * __builtin_popcountll(m);
+    int rank = 0;  // of the sequence of m's lowest bit in the window
+    for (; item < end; item += NW) {
+      const int r = (item - first) / per, k = item - first - r * per;
+      for (; rank < r; ++rank) m &= m - 1;
+      const int b = base + __builtin_ctzll(m), hh = k / F, f = k % F;
+      const int start = step_len(a, b) - 1, q = f % (F / 2);
+      int li = lane;  // opaque: lane addresses formed per item, not hoisted and spilled
+      asm volatile("" : "+v"(li));
+      if (f >= F / 2)
+        append_slice<HD, true, true>(g, a.wr, b, hh, q, start, 1, li, publish);
+      else
+        append_slice<HD, false, true>(g, a.wr, b, hh, q, start, 1, li, publish);
+      done = F * (b * NKV + hh) + f;
+      tf = __builtin_amdgcn_s_memrealtime();
     }
-    rank0 = rank;
+    first = end;
+  }
+  if (done >= 0) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    publish();
   }
   constexpr int V16 = HD / 8;
   const AppendArgs& w = a.wr;
@@ -1522,6 +1323,200 @@ __device__ __attribute__((always_inline)) inline uint64_t step_writer(const Kivi
   return tf - t0;
 }
 
+// Tiles [t_beg, t_fin) of a segment (sequence b, kv head h; ov quantised
+// tokens, n in all) by one wavefront, into st: its quantised groups through
+// the LDS ring, then its fp16 residual tiles.  FUSED: `aging` says that this
+// launch ages a group out of the sequence; the new group (tile g_age) and the
+// residual rows are then read with device-scope loads after wait_new(), and
+// residual row new_row (>= 0) comes from NEW_K / NEW_V.
+template <int HD, int P, bool PACK, bool FUSED, class Wait, class Progress>
+__device__ __attribute__((always_inline)) inline void decode_tiles(
+    const KiviGeo& g, const DecodeArgs& a, StageBuf<HD>* ring, uint16_t* qrows, const Nibble& nb,
+    float sscale, int lane, int b, int h, int ov, int n, int t_beg, int t_fin, int g_age,
+    int new_row, bool aging, WaveState<HD>& st, Wait& wait_new, Progress& progress,
+    uint64_t& t_first) {
+  using C = Cfg<HD, P>;
+  constexpr int KS = C::KS, CPL = C::CPL;
+  constexpr int L = stage_loads<HD>(), S = stages<HD, PACK>();
+  constexpr int QROW = HD + 8;
+  // lane-derived values per segment, not hoisted into the whole run
+  if constexpr (FUSED) asm volatile("" : "+v"(lane));
+  const int c = lane & 15, j = lane >> 4;
+  const int G = g.gqa, NKV = g.nkv;
+  const bool sum_col = sum_lane<HD>(c);
+
+  // ---- quantised groups: a ring of S LDS stages, S - 1 in flight ----
+  const int tq_end = min(t_fin, ov / kGroup);
+  // read-only for the whole launch: the constant address space lets the
+  // wave-uniform page reads be scalar loads (lgkmcnt, not vmcnt)
+  const __attribute__((address_space(4))) int32_t* bt =
+      (const __attribute__((address_space(4))) int32_t*)(a.block_tables +
+                                                         (int64_t)b * a.bt_stride);
+  const StageBases sb = stage_bases<HD, P>(a, NKV, h, lane);
+  auto page = [&](int tile, int k) -> uint32_t {
+    return (uint32_t)bt[tile * C::PPG + (C::PPG == 2 ? k : 0)];
+  };
+  uint32_t n0 = 0, n1 = 0;  // pages of group i + S - 1, read one group early
+  // The counts below see only this segment's DMAs.  The builtin, not asm:
+  // the compiler then knows that no load of its own is pending, and does not
+  // put a wait for one (and so for the DMAs ahead) into the group loop
+  // (8% of the fused HD 64 kernel for G > 8), whatever path leads here.
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  asm volatile("" ::: "memory");
+  if (t_beg < tq_end) {
+    if constexpr (FUSED) {
+      if (g_age >= t_beg && g_age < t_beg + S - 1 && g_age < tq_end) wait_new();
+    }
+#pragma unroll
+    for (int k = 0; k < S - 1; ++k)
+      if (t_beg + k < tq_end) {
+        if (FUSED && t_beg + k == g_age)
+          load_stage<HD, P, true>(&ring[k], sb, page(t_beg + k, 0), page(t_beg + k, 1), lane);
+        else
+          load_stage<HD, P>(&ring[k], sb, page(t_beg + k, 0), page(t_beg + k, 1), lane);
+      }
+    if (t_beg + S - 1 < tq_end) {
+      n0 = page(t_beg + S - 1, 0);
+      n1 = page(t_beg + S - 1, 1);
+    }
+  }
+
+  // ---- Q operands and softmax state (the loads overlap the first DMAs) ----
+  SegCtx<HD> q;
+  const uint16_t* qh = a.q + (int64_t)b * a.q_stride + (int64_t)h * G * HD;
+  // lane offsets from an opaque lane id (hoisted out of the segment loop,
+  // they would hold 64-bit registers through the whole run)
+  int lq = lane;
+  asm volatile("" : "+v"(lq));
+  const int hq = PACK ? (lq & 7) : (lq & 15);  // packed: columns c and c + 8 share head c
+  const int jq = lq >> 4;
+  uint16_t* qrow = &qrows[hq * QROW + jq * (HD / 4)];
+  q.qn = (const uint8_t*)qrow;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (hq < G) {
+      v = *(const u32x4*)(qh + hq * HD + jq * (HD / 4) + 8 * ks);
+      *(u32x4*)(qrow + 8 * ks) = v;  // the same words from columns c and c + 8
+    }
+    const half8_t div = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)0.0625f, (_Float16)0.0625f,
+                         (_Float16)1.0f, (_Float16)1.0f, (_Float16)0.0625f, (_Float16)0.0625f};
+    q.qp[ks] = as_h8(perm_pairs(v)) * div;
+  }
+#pragma unroll
+  for (int nt = 0; nt < CPL; ++nt) st.o[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  st.ob = floatx4{0.f, 0.f, 0.f, 0.f};
+  st.m = -1.0e30f;
+
+  const int r_beg = max(t_beg, ov / kGroup);  // first fp16 residual tile
+  if (t_beg < tq_end) {
+    const LaneMap lm = lane_map<HD, P>(lane);
+    int slot = 0;
+    for (int i = t_beg; i < tq_end; ++i) {
+      const int ahead = slot == 0 ? S - 1 : slot - 1;  // (slot + S - 1) % S
+      if (i + S - 1 < tq_end) {
+        if (FUSED && i + S - 1 == g_age) {
+          wait_new();
+          load_stage<HD, P, true>(&ring[ahead], sb, n0, n1, lane);
+        } else {
+          load_stage<HD, P>(&ring[ahead], sb, n0, n1, lane);
+        }
+        if (i + S < tq_end) {
+          n0 = page(i + S, 0);
+          n1 = page(i + S, 1);
+        }
+        wait_vm<(S - 1) * L>();
+      } else {
+        wait_stages<L, S>(tq_end - 1 - i);
+      }
+      if (a.stamps && t_first == 0) t_first = __builtin_amdgcn_s_memrealtime();
+      const VData vd = load_v<HD, P>(&ring[slot], lm);
+      const half8_t pa = qk_softmax<HD, P, PACK>(st, q, &ring[slot], lm, nb, sscale, lane);
+      st.ob = mfma(pa, as_h8(vd.vz4), st.ob);  // sum_t P z_t
+      pv_group<HD>(st, pa, vd, nb, big_scales(vd), false, PStash(nullptr));
+      // the range test comes last, so the steps above stay one block for
+      // the scheduler (a branch between them costs the common case ~15%)
+      if (__builtin_expect(wide_group<HD>(&ring[slot], lane), 0))
+        exact_fix_group<HD, P, PACK>(st, q, &ring[slot], lm, nb, sscale, lane, pa, vd);
+      slot = slot == S - 1 ? 0 : slot + 1;
+      progress(1);
+    }
+  }
+
+  // ---- fp16 residual tiles (all loads of a tile issued before its first use) ----
+  if constexpr (FUSED) {
+    if (aging && r_beg < t_fin) wait_new();
+  }
+  for (int i = r_beg; i < t_fin; ++i) {
+    ResTile<HD> cur =
+        (FUSED && aging) ? load_res<HD, FUSED, true>(a, g, b, h, ov, n, i, lane, new_row)
+                         : load_res<HD, FUSED, false>(a, g, b, h, ov, n, i, lane, new_row);
+    const int tn = min(kGroup, n - i * kGroup);  // 0 only for an empty sequence
+    floatx4 sres[2];
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+      sres[tt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) sres[tt] = mfma(as_h8(cur.kv[tt][ks]), q.n(ks), sres[tt]);
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii)
+        if (8 * j + 4 * tt + ii >= tn) sres[tt][ii] = -INFINITY;
+    }
+    // rows past the end carry P = 0 but must not carry NaN/Inf garbage
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      if (8 * j + r >= tn) cur.vr[r] = typename ResTile<HD>::vrow_t(0u);
+    // P also goes to LDS in fp32 (slot 0 is idle: every stage DMA has
+    // landed), for the exact correction of values above kFastRange
+    const PStash ps(ring[0].k);
+    const half8_t prh = softmax_tile<HD>(st, sres[0], sres[1], sscale, 0.0f, j, true, ps);
+    half2_t vmax = {(_Float16)0.0f, (_Float16)0.0f};
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int e = 0; e < (int)(sizeof(cur.vr[0]) / 4); ++e)
+        vmax = __builtin_elementwise_max(vmax, __builtin_elementwise_abs(as_h2(cur.vr[r][e])));
+    const bool wide = __builtin_amdgcn_ballot_w64((float)vmax[0] > kFastRange ||
+                                                  (float)vmax[1] > kFastRange) != 0;
+    // B operand of output columns nt: the tile rows' channels 16 nt + c
+    auto cols = [&](int nt) {
+      u32x4 vb;
+#pragma unroll
+      for (int qq = 0; qq < 4; ++qq) {
+        const uint32_t va = cur.vr[2 * qq][nt >> 1], vb2 = cur.vr[2 * qq + 1][nt >> 1];
+        vb[qq] = (nt & 1) ? __builtin_amdgcn_perm(vb2, va, 0x07060302u)
+                          : __builtin_amdgcn_perm(vb2, va, 0x05040100u);
+      }
+      return as_h8(vb);
+    };
+    // A residual tile (a few per segment, not the hot loop) takes one
+    // arithmetic or the other, chosen before its PV step: a correction
+    // after the fp16 step would turn an infinite value into inf - inf.
+    if (__builtin_expect(wide, 0)) {  // fp32 P against the (exact) fp16 values
+#pragma unroll
+      for (int nt = 0; nt < CPL; ++nt) {
+        const half8_t vh = cols(nt);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) st.o[nt] = mfma32(ps.get(i), (float)vh[i], st.o[nt]);
+      }
+      // Sigma P into the sum columns; the column test is redone from an
+      // opaque lane id, not kept live
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const float one = sum_lane<HD>(ln & 15) ? 1.0f : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) st.ob = mfma32(ps.get(i), one, st.ob);
+    } else {
+#pragma unroll
+      for (int nt = 0; nt < CPL; ++nt) st.o[nt] = mfma(prh, cols(nt), st.o[nt]);
+      const uint32_t one2 = sum_col ? 0x3C003C00u : 0u;  // Sigma P into the sum columns
+      st.ob = mfma(prh, as_h8(u32x4{one2, one2, one2, one2}), st.ob);
+    }
+    progress(kResidualUnits);
+  }
+}
+
 // One run of the stream: units [x0, x1) of the concatenated (sequence, kv
 // head) streams, starting in sequence sp.b.  `first_seg` with first_* gives
 // the first segment's window when the caller has it already.  Partials of cut
@@ -1532,10 +1527,7 @@ __device__ __attribute__((always_inline)) inline uint64_t stream_run(
     const KiviGeo& g, const DecodeArgs& a, StageBuf<HD>* ring, uint16_t* qrows, const Nibble& nb,
     float sscale, int lane, int64_t x0, int64_t x1, SeqSpan sp, bool first_seg, int first_T,
     int first_ov, int first_n, int w) {
-  using C = Cfg<HD, P>;
-  constexpr int KS = C::KS, CPL = C::CPL;
-  constexpr int L = stage_loads<HD>(), S = stages<HD, PACK>();
-  constexpr int QROW = HD + 8;
+  constexpr int CPL = HD / 16;
   const int c = lane & 15, j = lane >> 4;
   const int G = g.gqa, NKV = g.nkv;
   const bool sum_col = sum_lane<HD>(c);
@@ -1660,170 +1652,9 @@ __device__ __attribute__((always_inline)) inline uint64_t stream_run(
         // and residual rows are read with device-scope loads (COH)
       };
 
-      // ---- quantised groups: a ring of S LDS stages, S - 1 in flight ----
-      const int tq_end = min(t_fin, ov / kGroup);
-      // read-only for the whole launch: the constant address space lets the
-      // wave-uniform page reads be scalar loads (lgkmcnt, not vmcnt)
-      const __attribute__((address_space(4))) int32_t* bt =
-          (const __attribute__((address_space(4))) int32_t*)(a.block_tables +
-                                                             (int64_t)b * a.bt_stride);
-      const StageBases sb = stage_bases<HD, P>(a, NKV, h, lane);
-      auto page = [&](int tile, int k) -> uint32_t {
-        return (uint32_t)bt[tile * C::PPG + (C::PPG == 2 ? k : 0)];
-      };
-      uint32_t n0 = 0, n1 = 0;  // pages of group i + S - 1, read one group early
-      if (t_beg < tq_end) {
-        if constexpr (FUSED) {
-          if (g_age >= t_beg && g_age < t_beg + S - 1 && g_age < tq_end) wait_new();
-        }
-        wait_vm<0>();  // the counts below see only this segment's DMAs
-#pragma unroll
-        for (int k = 0; k < S - 1; ++k)
-          if (t_beg + k < tq_end)
-            if (FUSED && t_beg + k == g_age)
-              load_stage<HD, P, true>(&ring[k], sb, page(t_beg + k, 0), page(t_beg + k, 1), lane);
-            else
-              load_stage<HD, P>(&ring[k], sb, page(t_beg + k, 0), page(t_beg + k, 1), lane);
-        if (t_beg + S - 1 < tq_end) {
-          n0 = page(t_beg + S - 1, 0);
-          n1 = page(t_beg + S - 1, 1);
-        }
-      }
-
-      // ---- Q operands and softmax state (the loads overlap the first DMAs) ----
-      SegCtx<HD> q;
-      const uint16_t* qh = a.q + (int64_t)b * a.q_stride + (int64_t)h * G * HD;
-      // lane offsets from an opaque lane id (hoisted out of the segment loop,
-      // they would hold 64-bit registers through the whole run)
-      int lq = lane;
-      asm volatile("" : "+v"(lq));
-      const int hq = PACK ? (lq & 7) : (lq & 15);  // packed: columns c and c + 8 share head c
-      const int jq = lq >> 4;
-      uint16_t* qrow = &qrows[hq * QROW + jq * (HD / 4)];
-      q.qn = (const uint8_t*)qrow;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (hq < G) {
-          v = *(const u32x4*)(qh + hq * HD + jq * (HD / 4) + 8 * ks);
-          *(u32x4*)(qrow + 8 * ks) = v;  // the same words from columns c and c + 8
-        }
-        const half8_t div = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)0.0625f, (_Float16)0.0625f,
-                             (_Float16)1.0f, (_Float16)1.0f, (_Float16)0.0625f, (_Float16)0.0625f};
-        q.qp[ks] = as_h8(perm_pairs(v)) * div;
-      }
       WaveState<HD> st;
-#pragma unroll
-      for (int nt = 0; nt < CPL; ++nt) st.o[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-      st.ob = floatx4{0.f, 0.f, 0.f, 0.f};
-      st.m = -1.0e30f;
-
-      const int r_beg = max(t_beg, ov / kGroup);  // first fp16 residual tile
-      if (t_beg < tq_end) {
-        const LaneMap lm = lane_map<HD, P>(lane);
-        int slot = 0;
-        for (int i = t_beg; i < tq_end; ++i) {
-          const int ahead = slot == 0 ? S - 1 : slot - 1;  // (slot + S - 1) % S
-          if (i + S - 1 < tq_end) {
-            if (FUSED && i + S - 1 == g_age) {
-              wait_new();
-              load_stage<HD, P, true>(&ring[ahead], sb, n0, n1, lane);
-            } else {
-              load_stage<HD, P>(&ring[ahead], sb, n0, n1, lane);
-            }
-            if (i + S < tq_end) {
-              n0 = page(i + S, 0);
-              n1 = page(i + S, 1);
-            }
-            wait_vm<(S - 1) * L>();
-          } else {
-            wait_stages<L, S>(tq_end - 1 - i);
-          }
-          if (a.stamps && t_first == 0) t_first = __builtin_amdgcn_s_memrealtime();
-          const VData vd = load_v<HD, P>(&ring[slot], lm);
-          const half8_t pa = qk_softmax<HD, P, PACK>(st, q, &ring[slot], lm, nb, sscale, lane);
-          st.ob = mfma(pa, as_h8(vd.vz4), st.ob);  // sum_t P z_t
-          pv_group<HD>(st, pa, vd, nb, big_scales(vd), false, PStash(nullptr));
-          // the range test comes last, so the steps above stay one block for
-          // the scheduler (a branch between them costs the common case ~15%)
-          if (__builtin_expect(wide_group<HD>(&ring[slot], lane), 0))
-            exact_fix_group<HD, P, PACK>(st, q, &ring[slot], lm, nb, sscale, lane, pa, vd);
-          slot = slot == S - 1 ? 0 : slot + 1;
-          progress(1);
-        }
-      }
-
-      // ---- fp16 residual tiles (all loads of a tile issued before its first use) ----
-      if constexpr (FUSED) {
-        if (aging && r_beg < t_fin) wait_new();
-      }
-      for (int i = r_beg; i < t_fin; ++i) {
-        ResTile<HD> cur =
-            (FUSED && aging) ? load_res<HD, FUSED, true>(a, g, b, h, ov, n, i, lane, new_row)
-                             : load_res<HD, FUSED, false>(a, g, b, h, ov, n, i, lane, new_row);
-        const int tn = min(kGroup, n - i * kGroup);  // 0 only for an empty sequence
-        floatx4 sres[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-          sres[tt] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks) sres[tt] = mfma(as_h8(cur.kv[tt][ks]), q.n(ks), sres[tt]);
-#pragma unroll
-          for (int ii = 0; ii < 4; ++ii)
-            if (8 * j + 4 * tt + ii >= tn) sres[tt][ii] = -INFINITY;
-        }
-        // rows past the end carry P = 0 but must not carry NaN/Inf garbage
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-          if (8 * j + r >= tn) cur.vr[r] = typename ResTile<HD>::vrow_t(0u);
-        // P also goes to LDS in fp32 (slot 0 is idle: every stage DMA has
-        // landed), for the exact correction of values above kFastRange
-        const PStash ps(ring[0].k);
-        const half8_t prh = softmax_tile<HD>(st, sres[0], sres[1], sscale, 0.0f, j, true, ps);
-        half2_t vmax = {(_Float16)0.0f, (_Float16)0.0f};
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-#pragma unroll
-          for (int e = 0; e < (int)(sizeof(cur.vr[0]) / 4); ++e)
-            vmax = __builtin_elementwise_max(vmax, __builtin_elementwise_abs(as_h2(cur.vr[r][e])));
-        const bool wide = __builtin_amdgcn_ballot_w64((float)vmax[0] > kFastRange ||
-                                                      (float)vmax[1] > kFastRange) != 0;
-        // B operand of output columns nt: the tile rows' channels 16 nt + c
-        auto cols = [&](int nt) {
-          u32x4 vb;
-#pragma unroll
-          for (int qq = 0; qq < 4; ++qq) {
-            const uint32_t va = cur.vr[2 * qq][nt >> 1], vb2 = cur.vr[2 * qq + 1][nt >> 1];
-            vb[qq] = (nt & 1) ? __builtin_amdgcn_perm(vb2, va, 0x07060302u)
-                              : __builtin_amdgcn_perm(vb2, va, 0x05040100u);
-          }
-          return as_h8(vb);
-        };
-        // A residual tile (a few per segment, not the hot loop) takes one
-        // arithmetic or the other, chosen before its PV step: a correction
-        // after the fp16 step would turn an infinite value into inf - inf.
-        if (__builtin_expect(wide, 0)) {  // fp32 P against the (exact) fp16 values
-#pragma unroll
-          for (int nt = 0; nt < CPL; ++nt) {
-            const half8_t vh = cols(nt);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) st.o[nt] = mfma32(ps.get(i), (float)vh[i], st.o[nt]);
-          }
-          // Sigma P into the sum columns; the column test is redone from an
-          // opaque lane id, not kept live
-          int ln = lane;
-          asm volatile("" : "+v"(ln));
-          const float one = sum_lane<HD>(ln & 15) ? 1.0f : 0.0f;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) st.ob = mfma32(ps.get(i), one, st.ob);
-        } else {
-#pragma unroll
-          for (int nt = 0; nt < CPL; ++nt) st.o[nt] = mfma(prh, cols(nt), st.o[nt]);
-          const uint32_t one2 = sum_col ? 0x3C003C00u : 0u;  // Sigma P into the sum columns
-          st.ob = mfma(prh, as_h8(u32x4{one2, one2, one2, one2}), st.ob);
-        }
-        progress(kResidualUnits);
-      }
+      decode_tiles<HD, P, PACK, FUSED>(g, a, ring, qrows, nb, sscale, lane, b, h, ov, n, t_beg, t_fin,
+                                       g_age, new_row, aging, st, wait_new, progress, t_first);
 
       // ---- segment output: O directly, or a partial for the merge workgroups ----
       // row sums: Sigma P of O row 4j + i sits in the sum column C1 of row
@@ -1925,14 +1756,9 @@ __device__ __attribute__((always_inline)) inline uint64_t stream_run(
 
 
 
-// The per-query kernels (PQ) keep one more run's state live across their run
-// loop, which at three waves per SIMD spills; they run with the register
-// budget of two (the v1 symbols decode one sequence, or the causal prefixes
-// of one, far from filling the device).
-template <int HD, int P, bool PACK, bool PQ, bool FUSED>
+template <int HD, int P, bool PACK, bool FUSED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
-    PQ ? 1 : min_waves_per_simd<HD, PACK>()))) void kivi_decode_stream_kernel(KiviGeo g,
-                                                                              DecodeArgs a) {
+    min_waves_per_simd<HD, PACK>()))) void kivi_decode_stream_kernel(KiviGeo g, DecodeArgs a) {
   constexpr int S = stages<HD, PACK>();
   static_assert(S >= 2 && S <= 4, "wait_stages covers up to 3 stages in flight");
   __shared__ __attribute__((aligned(16))) StageBuf<HD> ring[S];
@@ -1962,30 +1788,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
   if (bid >= a.waves) {
     // profiling: the ticks from the merge's start to the end of its last wait
     // (bits 32-55) and the load rounds after that wait (bits 56-61)
-    const uint64_t t_wait = merge_segments<HD, PACK, PQ, FUSED>(g, a, lane);
+    const uint64_t t_wait = merge_segments<HD, PACK, FUSED>(g, a, lane);
     write_stamp(a, t_start, t_wait << 32, lane);
-    return;
-  }
-  if constexpr (PQ) {
-    const Nibble nb;
-    // the ones block of every stage (the DMAs never write it)
-    if (lane < 32) {
-#pragma unroll
-      for (int s_ = 0; s_ < S; ++s_) ((uint32_t*)ring[s_].ones)[lane] = 0x3C003C00u;
-    }
-    // rows past G are read as zeros by the columns that carry no head
-    for (int i = lane; i < (int)(sizeof(qrows) / 16); i += 64)
-      ((u32x4*)qrows)[i] = u32x4{0u, 0u, 0u, 0u};
-    const float sscale = 1.4426950408889634f / __builtin_sqrtf((float)HD);  // log2(e)/sqrt(HD)
-    for (int64_t r = bid;; r += a.waves) {
-      const RunLoc rl = locate_run(g, a, r, lane);
-      if (rl.q < 0) break;
-      const int64_t TTq = (int64_t)g.nkv * rl.units, wl = r - rl.r0;
-      const int64_t x0 = wl * TTq / rl.runs, x1 = (wl + 1) * TTq / rl.runs;
-      if (x0 >= x1) continue;
-      stream_run<HD, P, PACK, false>(g, a, ring, qrows, nb, sscale, lane, x0, x1,
-                                     SeqSpan{rl.q, 0, rl.units}, false, 0, 0, 0, (int)r);
-    }
     return;
   }
   const int G = g.gqa, NKV = g.nkv;
@@ -1998,10 +1802,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
     lane_T = seq_tiles(g, a, lane, &lane_ov, &lane_n);
     lane_U = lane_ov / kGroup + kResidualUnits * (lane_T - lane_ov / kGroup);
   }
-  const int lane_incl = wave_incl_scan(lane_U, lane);
+  const int lane_incl = wave_incl_scan(lane_U);
   const int64_t TT = one_pass ? (int64_t)NKV * __builtin_amdgcn_readlane(lane_incl, 63)
                               : stream_units(g, a, lane);
-  const int64_t W = stream_waves(TT, a.waves, true);
+  const int64_t W = stream_waves(TT, a.waves);
   const int w = bid;
   const int64_t nw = FUSED ? a.writer_waves : 0;
   if (w >= W) return;
@@ -2043,31 +1847,455 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
   write_stamp(a, t_start, (uint64_t)(x1 - x0) | ((t_first ? t_first - t_start : 0) << 32), lane);
 }
 
+// ---- calls of few segments: one workgroup per chunk of a segment ----
+//
+// With at most one (sequence, kv head) segment per CU the stream above cuts
+// every segment among many wavefronts, and the merge of their partials, two or
+// eight per memory round, outlasts the decode: 65 pieces per segment in a
+// 16k-token sequence at 8 kv heads took 36 of 52 us.  Here a workgroup of nw
+// wavefronts takes a chunk of one segment: its wavefronts decode nw equal runs of the
+// chunk's units and their partials meet in LDS.  A segment of one chunk is
+// written whole; the chunks of a longer one go to the workspace, and whichever
+// workgroup stores its chunk last folds them all, in chunk order, with the
+// loads of eight chunks in flight.
+//
+// Last: a workgroup's partial is complete at the point of coherence
+// before its flag (the launch's epoch) is stored, and its flag before it reads the
+// segment's other flags, so of any two workgroups the later sees the earlier's
+// flag: at least one sees all.  It clears them (a replayed graph repeats the
+// epoch); one that sees a cleared flag leaves, and two that both see all write
+// the same bits.  Nothing waits for another workgroup.
+//
+// The fused step's write is the last chunk's: it holds the new group and the
+// residual rows whenever a group ages out (its first unit is lowered to the new
+// group's), so a barrier orders the write before the reads.
+//
+// Measured against the stream, a pass among others: 32 sequences of 4096 tokens
+// (32 / 8 heads, HD 128) 51.0 -> 39.6 us, one of 16001 with half its pages evicted
+// 51.7 -> 16.8, 80 of 101 to 6007 (32 / 2 heads) 62.9 -> 33.3, 16 of 2048 (14 / 2,
+// HD 64) 16.8 -> 13.1, a v1 write and query at 2900 28.9 -> 17.0, 31 v1 queries at
+// 2048 82 -> 47.  What is left at the small end is latency: 2.2 us to the plan (the
+// lengths' round), 2.3 for the table and the first group, 1.1 per unit and
+// wavefront, 1 for the fold, 4 for a cut.
+
+// Chunks a segment of `units` units is cut into: at most `cu` units each, one
+// where the segment has no more than `whole`.
+__device__ inline int chunk_count(int units, int cu, int whole) {
+  return units <= whole ? 1 : (units + cu - 1) / cu;
+}
+
+// Sequences a call of the chunk kernel may hold: at most one segment per CU.
+constexpr int kChunkWindows = 4;  // of 64 sequences, one per lane
+
+// Units per chunk of a whole call: the fewest that make no more chunks than
+// workgroups are resident at once (one more chunk would be a second round for
+// all), but at least a.chunk_units.  The count falls as the units grow, so it is
+// bracketed by doubling and halved down to 1/16.  `units`: the lane's sequences'.
+__device__ inline int chunk_units(const KiviGeo& g, const DecodeArgs& a,
+                                  const int (&units)[kChunkWindows]) {
+  const int slots = max(a.chunk_slots, a.batch * g.nkv);
+  auto fits = [&](int cu) {
+    int c = 0;
+#pragma unroll
+    for (int w = 0; w < kChunkWindows; ++w)
+      if (64 * w < a.batch) c += units[w] > 0 ? chunk_count(units[w], cu, a.chunk_whole) : 0;
+    return wave_sum_i(c) * g.nkv <= slots;
+  };
+  int tot = 0;
+#pragma unroll
+  for (int w = 0; w < kChunkWindows; ++w) tot += units[w];
+  tot = wave_sum_i(tot) * g.nkv;
+  int lo = max(a.chunk_units, (tot + slots - 1) / slots);
+  if (fits(lo)) return lo;
+  int hi = 2 * lo;
+  while (!fits(hi)) {  // ends: with one chunk per segment the slots suffice
+    lo = hi;
+    hi *= 2;
+  }
+  while (hi - lo > lo / 16 + 1) {
+    const int mid = (lo + hi) / 2;
+    if (fits(mid))
+      hi = mid;
+    else
+      lo = mid;
+  }
+  return hi;
+}
+
+// Dynamic LDS: per wavefront its ring and Q rows (its partial takes the ring's
+// place when its run is done), then one control word.
+template <int HD, bool PACK>
+constexpr int coop_wave_lds() {
+  return stages<HD, PACK>() * (int)sizeof(StageBuf<HD>) + (PACK ? 8 : 16) * (HD + 8) * 2;
+}
+// The most wavefronts of a workgroup: what a CU's 160 KiB of LDS and the
+// registers hold.
+template <int HD, bool PACK>
+constexpr int coop_max_waves() {
+  return HD == 128 && !PACK ? 8 : 12;
+}
+
+template <int HD, int P, bool PACK, bool FUSED>
+__global__ __launch_bounds__(64 * (coop_max_waves<HD, PACK>())) void kivi_decode_chunk_kernel(
+    KiviGeo g, DecodeArgs a) {
+  constexpr int S = stages<HD, PACK>(), CPL = HD / 16, QROW = HD + 8;
+  constexpr int C1 = kGroup / CPL - 1;  // a sum column
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  uint8_t* mine = lds + wv * coop_wave_lds<HD, PACK>();
+  StageBuf<HD>* ring = (StageBuf<HD>*)mine;
+  uint16_t* qrows = (uint16_t*)(mine + S * sizeof(StageBuf<HD>));
+  uint32_t* ctl = (uint32_t*)(lds + nw * coop_wave_lds<HD, PACK>());
+  const uint64_t t_start = a.stamps ? __builtin_amdgcn_s_memrealtime() : 0;
+  uint64_t t_first = 0, units_done = 0;  // profiling
+  const int G = g.gqa, NKV = g.nkv;
+  const Nibble nb;
+  const float sscale = 1.4426950408889634f / __builtin_sqrtf((float)HD);  // log2(e)/sqrt(HD)
+  // rows past G are read as zeros by the columns that carry no head
+  for (int i = lane; i < (PACK ? 8 : 16) * QROW / 8; i += 64) ((u32x4*)qrows)[i] = u32x4{0u, 0u, 0u, 0u};
+
+  // the windows of the first 64 sequences, one per lane
+  struct Window {
+    int ov, n, units;
+  };
+  auto window = [&](int bb) {
+    Window w{0, 0, 0};
+    if (bb < a.batch) {
+      const int T = seq_tiles(g, a, bb, &w.ov, &w.n), nq = w.ov / kGroup;
+      w.units = nq + kResidualUnits * (T - nq);
+    }
+    return w;
+  };
+  Window first = window(lane);
+  // per query (the v1 symbols): the caller's constant, so that a query is cut by
+  // its own length alone, in a call with others as by itself
+  int cu = a.chunk_units;
+  if (!a.per_query) {
+    int units[kChunkWindows] = {first.units, 0, 0, 0};
+#pragma unroll
+    for (int w = 1; w < kChunkWindows; ++w)
+      if (64 * w < a.batch) units[w] = window(64 * w + lane).units;
+    cu = chunk_units(g, a, units);
+  }
+  for (int x = blockIdx.x;; x += gridDim.x) {
+    // the chunk x: sequence by sequence, kv head by kv head, chunk by chunk
+    int b = -1, U = 0, cnt = 0, rel = 0, before = 0, ov = 0, n = 0;
+    for (int base = 0; base < a.batch; base += 64) {
+      const Window w = base == 0 ? first : window(base + lane);
+      const int cl = w.units > 0 ? NKV * chunk_count(w.units, cu, a.chunk_whole) : 0;
+      const int incl = wave_incl_scan(cl);
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(before + incl > x);
+      if (hit) {
+        const int f = __builtin_ctzll(hit);
+        b = base + f;
+        U = __builtin_amdgcn_readlane(w.units, f);
+        ov = __builtin_amdgcn_readlane(w.ov, f);
+        n = __builtin_amdgcn_readlane(w.n, f);
+        cnt = chunk_count(U, cu, a.chunk_whole);
+        rel = x - before - (__builtin_amdgcn_readlane(incl, f) - cnt * NKV);
+        break;
+      }
+      before += __builtin_amdgcn_readlane(incl, 63);
+    }
+    if (b < 0) break;
+    const int h = rel / cnt, ci = rel - h * cnt;
+    const int nq = ov / kGroup;
+    int u0 = (int)((int64_t)ci * U / cnt), u1 = (int)((int64_t)(ci + 1) * U / cnt);
+
+    // ---- fused step: the last chunk writes ----
+    int g_age = 0x7fffffff, new_row = -1, Lb = 0;
+    bool ages = false;
+    if constexpr (FUSED) {
+      Lb = step_len(a, b);
+      ages = step_ages(g, Lb);
+      if (ages) {
+        if (ov == split_old_tokens(Lb, g.residual)) g_age = nq - 1;
+        const int keep = max(nq - 1, 0);  // the new group and all residual tiles in the last chunk
+        if (ci > 0) u0 = min(u0, keep);
+        if (ci < cnt - 1) u1 = min(u1, keep);
+        if (ci == cnt - 1) {
+          constexpr int F = step_flags<HD>();
+          for (int f = wv; f < F; f += nw) {
+            int li = lane;  // opaque: lane addresses formed per item
+            asm volatile("" : "+v"(li));
+            if (f >= F / 2)
+              append_slice<HD, true, true>(g, a.wr, b, h, f - F / 2, Lb - 1, 1, li, [] {});
+            else
+              append_slice<HD, false, true>(g, a.wr, b, h, f, Lb - 1, 1, li, [] {});
+          }
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+        }
+      } else if (Lb == n && n > ov) {
+        new_row = n - ov - 1;
+      }
+    }
+
+    // ---- this wavefront's run of the chunk ----
+    const int ua = u0 + (int)((int64_t)(u1 - u0) * wv / nw),
+              ub = u0 + (int)((int64_t)(u1 - u0) * (wv + 1) / nw);
+    const int t_beg = tile_at(ua, nq), t_fin = tile_at(ub, nq);
+    // the ones block of every stage (the DMAs never write it; a partial may have)
+    if (lane < 32) {
+#pragma unroll
+      for (int s_ = 0; s_ < S; ++s_) ((uint32_t*)ring[s_].ones)[lane] = 0x3C003C00u;
+    }
+    WaveState<HD> st;
+    float* ml = (float*)mine;       // partial: (m, l) per head, 16 of them, then acc
+    float* acc = (float*)mine + 32;
+    static_assert(S * sizeof(StageBuf<HD>) >= (32 + (PACK ? 8 : 16) * HD) * sizeof(float), "partial");
+    if (t_beg < t_fin) {
+      auto no_wait = [] {};
+      // issue priority by progress, as in the stream kernel's runs
+      const int n_run = ub - ua, q1 = n_run / 2, q2 = 4 * n_run / 5, q3 = 19 * n_run / 20;
+      int done = 0, level = 3;
+      __builtin_amdgcn_s_setprio(3);
+      auto progress = [&](int units) {
+        done += units;
+        if (level == 3 && done >= q1) {
+          __builtin_amdgcn_s_setprio(2);
+          level = 2;
+        }
+        if (level == 2 && done >= q2) {
+          __builtin_amdgcn_s_setprio(1);
+          level = 1;
+        }
+        if (level == 1 && done >= q3) {
+          __builtin_amdgcn_s_setprio(0);
+          level = 0;
+        }
+      };
+      decode_tiles<HD, P, PACK, FUSED>(g, a, ring, qrows, nb, sscale, lane, b, h, ov, n, t_beg,
+                                       t_fin, g_age, new_row, ages, st, no_wait, progress,
+                                       t_first);
+      // ---- its partial to LDS (the ring is idle: every DMA has landed) ----
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int c = ln & 15, j = ln >> 4;
+      const bool sum_col = sum_lane<HD>(c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float left = __shfl(st.ob[i], ln - 1, 64);
+        const float z = sum_col ? left : st.ob[i];
+        if (4 * j + i < G) {
+          float* p = acc + (4 * j + i) * HD + CPL * c;
+#pragma unroll
+          for (int q4 = 0; q4 < CPL / 4; ++q4)
+            *(floatx4*)(p + 4 * q4) = floatx4{st.o[4 * q4][i] + z, st.o[4 * q4 + 1][i] + z,
+                                              st.o[4 * q4 + 2][i] + z, st.o[4 * q4 + 3][i] + z};
+          if (c == C1) ml[2 * (4 * j + i) + 1] = st.ob[i];  // Sigma P of head 4j + i
+        }
+      }
+      if (j == 0 && c < G) ml[2 * c] = st.m;
+    } else if (lane < G) {
+      ml[2 * lane] = -INFINITY;  // no tile: skipped below
+    }
+    __syncthreads();
+
+    // ---- the chunk: fold the wavefronts' partials in order ----
+    // an opaque thread id: addresses formed from here on are not computed (and
+    // spilled) before the tiles
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int ln = tid & 63;
+    // ---- fused step: a plain append, whose row no wavefront reads from the
+    // scratch, by the last wavefront (the fold below needs only the first few) ----
+    if constexpr (FUSED) {
+      const int r0 = Lb - 1 - split_old_tokens(Lb - 1, g.residual);
+      constexpr int V16 = HD / 8;
+      if (!ages && ci == cnt - 1 && Lb >= 1 && wv == nw - 1 && r0 < g.rs && ln < 2 * V16) {
+        const bool v = ln >= V16;
+        const int64_t at = (int64_t)h * g.rs * HD + (int64_t)r0 * HD + 8 * (ln % V16);
+        const uint16_t* nx = (v ? a.wr.new_v : a.wr.new_k) + (int64_t)b * a.wr.new_stride +
+                             (int64_t)h * HD + 8 * (ln % V16);
+        *(u32x4*)((v ? a.wr.v_scr : a.wr.k_scr) + (int64_t)b * a.wr.scr_stride + at) =
+            *(const u32x4*)nx;
+      }
+    }
+    const int n4 = G * HD / 4;
+    const bool whole = cnt == 1;
+    float* const out = a.out + (int64_t)b * a.out_stride + (int64_t)h * G * HD;
+    for (int e = tid; e < n4; e += blockDim.x) {
+      const int gi = 4 * e / HD;
+      const float* pm = (const float*)lds + 2 * gi;
+      const float* pa = (const float*)lds + 32 + 4 * e;
+      constexpr int W = coop_wave_lds<HD, PACK>() / 4, NW = coop_max_waves<HD, PACK>();
+      float M = -INFINITY, L = 0.0f;
+      floatx4 v = {0.f, 0.f, 0.f, 0.f};
+      // every read in flight at once; past the last wavefront the last again,
+      // with weight 0
+      uint64_t pml[NW];
+      floatx4 pv[NW];
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const int at = min(w, nw - 1) * W;
+        pml[w] = *(const uint64_t*)(pm + at);
+        pv[w] = *(const floatx4*)(pa + at);
+      }
+#pragma unroll
+      for (int w = 0; w < NW; ++w) M = fmaxf(M, lo_f(pml[w]));
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        // a wavefront without a tile left (-inf) and what lay in its ring
+        const bool on = w < nw && lo_f(pml[w]) != -INFINITY;
+        const float f = on ? __builtin_amdgcn_exp2f(lo_f(pml[w]) - M) : 0.0f;
+        L += on ? hi_f(pml[w]) * f : 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += on ? pv[w][i] * f : 0.0f;
+      }
+      if (whole) {
+        *(floatx4*)(out + 4 * e) = v * (1.0f / fmaxf(L, 1.0e-30f));
+      } else {
+        st_agent4(a.ws_acc + (int64_t)x * G * HD + 4 * e, v);
+        if (4 * e == gi * HD) st_agent(a.ws_ml + 2 * ((int64_t)x * G + gi), M, L);
+      }
+    }
+    if (!whole) {
+      // complete at the point of coherence before the flag
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      uint64_t* const flags = a.ws_flag + (x - ci);
+      if (wv == 0) {
+        uint64_t epoch = a.epoch;  // opaque: moved to registers here, not before the tiles
+        asm volatile("" : "+s"(epoch));
+        if (ln == 0)
+          __hip_atomic_store(flags + ci, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        bool all = true;
+        for (int k = ln; k < cnt; k += 64) all = all && ld_agent(flags + k) == epoch;
+        const bool poison = a.ws_poison && ld_agent(a.ws_poison) == kWorkspacePoison;
+        const bool last = __builtin_amdgcn_ballot_w64(!all) == 0;
+        // the forced time-out of the tests, and a workspace that an earlier
+        // launch's time-out poisoned: NaN, and reported
+        const bool bad = a.merge_skew != 0 || (last && poison);
+        if (last && !a.merge_skew)
+          for (int k = ln; k < cnt; k += 64)
+            __hip_atomic_store(flags + k, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (ln == 0) {
+          *ctl = bad ? 2u : last ? 1u : 0u;
+          if (bad) {
+            uint64_t mark = kWorkspacePoison;
+            asm volatile("" : "+s"(mark));
+            if (a.ws_poison)
+              __hip_atomic_store(a.ws_poison, mark, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+            if (a.status)
+              __hip_atomic_store(a.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+          }
+        }
+      }
+      __syncthreads();
+      const uint32_t what = *ctl;
+      if (what) {
+        for (int e = tid; e < n4; e += blockDim.x) {
+          const int gi = 4 * e / HD;
+          float M = -INFINITY, L = 0.0f;
+          floatx4 v = {0.f, 0.f, 0.f, 0.f};
+          constexpr int N = 8;  // chunks whose loads are in flight together
+          for (int k0 = 0; k0 < cnt; k0 += N) {
+            uint64_t pml[N];
+            floatx4 pv[N];
+#pragma unroll
+            for (int k = 0; k < N; ++k) {  // past the last: the last again, with weight 0
+              const int64_t at = (int64_t)(x - ci + min(k0 + k, cnt - 1)) * G;
+              pml[k] = ld_agent(a.ws_ml + 2 * (at + gi));
+              pv[k] = ld_agent4(a.ws_acc + at * HD + 4 * e);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int k = 0; k < N; ++k) keep(pv[k]);
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+              const float m = lo_f(pml[k]);
+              if (k0 + k >= cnt || m == -INFINITY) continue;
+              const float mn = fmaxf(M, m);
+              const float fo = __builtin_amdgcn_exp2f(M - mn), fn = __builtin_amdgcn_exp2f(m - mn);
+              v = v * fo + pv[k] * fn;
+              L = L * fo + hi_f(pml[k]) * fn;
+              M = mn;
+            }
+          }
+          *(floatx4*)(out + 4 * e) =
+              what == 2 ? floatx4{NAN, NAN, NAN, NAN} : v * (1.0f / fmaxf(L, 1.0e-30f));
+        }
+      }
+    }
+    units_done += u1 - u0;
+    if (!a.per_query) break;  // as many workgroups as chunks
+    __syncthreads();  // the rings are used again by the next chunk
+    int l2 = lane;    // the windows again, not kept through the chunk
+    asm volatile("" : "+v"(l2));
+    first = window(l2);
+  }
+  if (wv == 0)
+    write_stamp(a, t_start, units_done | ((t_first ? t_first - t_start : 0) << 32), lane);
+}
+
+template <int HD, int P, bool PACK, bool FUSED>
+static void launch_chunks(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream,
+                          hipEvent_t start, hipEvent_t stop) {
+  const unsigned lds = (unsigned)(a.chunk_waves * coop_wave_lds<HD, PACK>() + 16);
+  hipExtLaunchKernelGGL((kivi_decode_chunk_kernel<HD, P, PACK, FUSED>), dim3(a.chunk_grid),
+                        dim3(64 * a.chunk_waves), lds, stream, start, stop, 0, g, a);
+}
+
+template <int HD, int P, bool PACK>
+static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream,
+                       hipEvent_t start, hipEvent_t stop) {
+  if (a.chunk_waves > 0) {
+    if (a.fused)
+      launch_chunks<HD, P, PACK, true>(g, a, stream, start, stop);
+    else
+      launch_chunks<HD, P, PACK, false>(g, a, stream, start, stop);
+    return;
+  }
+  const dim3 grid(a.waves + a.merge_wgs);
+  const dim3 block(64);
+  if (a.fused)
+    hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, PACK, true>), grid, block, 0, stream,
+                          start, stop, 0, g, a);
+  else
+    hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, PACK, false>), grid, block, 0, stream,
+                          start, stop, 0, g, a);
+}
+
 template <int HD, int P>
 static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream,
                        hipEvent_t start, hipEvent_t stop) {
-  const dim3 grid(a.waves + a.merge_wgs);
-  const dim3 block(64);
-  if (a.writer_waves > 0) {
-    if (g.gqa <= 8)
-      hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, true, false, true>), grid, block, 0,
-                            stream, start, stop, 0, g, a);
-    else
-      hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, false, false, true>), grid, block,
-                            0, stream, start, stop, 0, g, a);
-  } else if (g.gqa <= 8 && a.per_query) {
-    hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, true, true, false>), grid, block, 0,
-                          stream, start, stop, 0, g, a);
-  } else if (g.gqa <= 8) {
-    hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, true, false, false>), grid, block, 0,
-                          stream, start, stop, 0, g, a);
-  } else if (a.per_query) {
-    hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, false, true, false>), grid, block, 0,
-                          stream, start, stop, 0, g, a);
-  } else {
-    hipExtLaunchKernelGGL((kivi_decode_stream_kernel<HD, P, false, false, false>), grid, block,
-                          0, stream, start, stop, 0, g, a);
-  }
+  if (g.gqa <= 8)
+    launch_one<HD, P, true>(g, a, stream, start, stop);
+  else
+    launch_one<HD, P, false>(g, a, stream, start, stop);
+}
+
+// Calls of at most one segment per CU go to the chunk kernel, and all of the v1
+// symbols', whose queries must decode to the same bits alone and together.
+//  - Whole calls take the largest workgroup a CU holds (twelve wavefronts, eight of
+//    the HD 128 kernel for G > 8): the fold in LDS costs 1 us whatever their number,
+//    a cut between workgroups 4 us.  So a segment of up to three units per wavefront
+//    (3 us) stays whole, and a longer one is cut down to one unit per
+//    wavefront where workgroups are free (2 and 3 units were 1 to 2 us slower for
+//    one 16k-token sequence and for 16 of 2048 tokens).
+//  - The v1 symbols take four wavefronts and 16 units: one 2900-token query is
+//    faster with fewer units (8: 15.8 us against 17.0 with its write; 32: 20.3),
+//    31 causal ones with more (47 us; 8: 65, 32: 41).
+ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_query, int cus) {
+  ChunkPlan p{};
+  const int most = g.hd == 128 && g.gqa > 8 ? 8 : 12;
+  const int64_t segs = (int64_t)batch * g.nkv;
+  if (!per_query && (segs > cus || batch > 64 * kChunkWindows)) return p;
+  p.waves = per_query ? 4 : most;
+  p.units = per_query ? 16 : most;
+  p.whole = per_query ? 0 : 3 * most;
+  const int64_t tiles = std::max<int64_t>(1, (max_tokens + kGroup - 1) / kGroup);
+  // a segment's units at most: R / 32 + 1 of its tiles are residual
+  const int64_t units = tiles + (kResidualUnits - 1) * (g.residual / kGroup + 1);
+  const int64_t per_segment = units <= p.whole ? 1 : (units + p.units - 1) / p.units;
+  if (per_query) p.per_query = (int)(g.nkv * per_segment);
+  p.slots = cus * (most / p.waves);
+  p.grid = (int)std::min<int64_t>(segs * per_segment, p.slots);
+  return p;
 }
 
 hipError_t launch_decode_mfma(const KiviGeo& g, const DecodeArgs& args, int batch,
@@ -2123,7 +2351,7 @@ static int resident_per_cu() {
   static int n = 0;
   if (n == 0) {
     int k = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, kivi_decode_stream_kernel<HD, P, PACK, false, false>,
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&k, kivi_decode_stream_kernel<HD, P, PACK, false>,
                                                      64, 0) != hipSuccess ||
         k < 1)
       k = 8;

@@ -58,7 +58,13 @@ struct DecodeArgs {
   int retained_pages = -1;  // >= 0: sparse-retained window (compact block table)
   uint32_t* status = nullptr;  // matrix-core kernel: set to 1 when a merge wait runs out
   uint64_t* ws_poison = nullptr;  // matrix-core kernel: the workspace's poison word
-  int per_query = 0;  // matrix-core kernel: cut each query's streams by its own length alone
+  // Chunk kernel (calls of few segments, and the v1 symbols): wavefronts per
+  // workgroup (0: the stream kernel), workgroups launched and resident at
+  // once, units per chunk (per_query: exactly, by each query's own length alone;
+  // else at least), units up to which a segment is one chunk.
+  int chunk_waves = 0, chunk_grid = 0, chunk_slots = 0, chunk_units = 0, chunk_whole = 0;
+  int per_query = 0;
+  int fused = 0;  // jacq_kivi_write_decode
   // Fused write + decode (jacq_kivi_write_decode): the writer's arrays (one
   // new token per sequence; its length before the write is seq_lens - 1), the
   // count of stream wavefronts at the front of the grid that do the writer's
@@ -106,6 +112,12 @@ hipError_t launch_decode_mfma(const KiviGeo& g, const DecodeArgs& a, int batch,
 // epoch no wavefront stores and gives up after `us` microseconds; 0 restores
 // normal operation.
 void set_test_merge_timeout_us(uint32_t us);
+// How the matrix-core decode cuts a call: waves > 0 selects the chunk kernel.
+struct ChunkPlan {
+  int waves, grid, slots, units, whole;
+  int per_query;  // per-query split: chunks of a query at most (all kv heads)
+};
+ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_query, int cus);
 // wavefronts the matrix-core decode launches on a device with `cus` CUs:
 // as many as are resident at once
 int decode_stream_waves(const KiviGeo& g, int cus);

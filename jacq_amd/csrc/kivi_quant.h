@@ -337,11 +337,13 @@ __device__ inline void group_pages(const KiviGeo& g, const AppendArgs& a, int b,
 // handled here.  What bounds it is latency (lengths, then rows and table,
 // then stores): every row of a one-group age-out at R <= 128 is loaded in one
 // round.
-template <int HD, bool IS_V, bool DEV>
+// landed() is called where everything the wavefront issued before this slice is
+// complete.
+template <int HD, bool IS_V, bool DEV, class Landed>
 __device__ __attribute__((always_inline)) inline void append_slice(const KiviGeo& g,
                                                                    const AppendArgs& a, int b,
                                                                    int h, int q, int start, int n,
-                                                                   int lane) {
+                                                                   int lane, Landed&& landed) {
   const AppendSpan sp(g, start, n);
   const int c = lane & 3, r = lane >> 2;
   uint16_t* xs = (IS_V ? a.v_scr : a.k_scr) + (int64_t)b * a.scr_stride + (int64_t)h * g.rs * HD +
@@ -363,7 +365,7 @@ __device__ __attribute__((always_inline)) inline void append_slice(const KiviGeo
     x[1] = row(16 + r);
   }
   // every load unconditional (past the last row it re-reads that row): under a
-  // per-lane branch the compiler waits for each before the next
+  // branch the compiler waits for each before the next
 #pragma unroll
   for (int k = 0; k < kPer; ++k) sh[k] = row(sp.D + min(r + 16 * k, sp.r1 - 1));
   for (int gi = 0; gi < ng; ++gi) {
@@ -384,6 +386,7 @@ __device__ __attribute__((always_inline)) inline void append_slice(const KiviGeo
       for (int k = 0; k < kPer; ++k) sh[k] = row(sp.D + min(base + r + 16 * k, sp.r1 - 1));
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (base == 0) landed();
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
       const int d = base + r + 16 * k;

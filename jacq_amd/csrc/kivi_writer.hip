@@ -59,16 +59,16 @@ __global__ __launch_bounds__(64 * (HD / kGroup)) void kivi_append_kernel(KiviGeo
   constexpr int WPB = HD / kGroup;
   const int b = blockIdx.y, x = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int start = a.start_lens ? a.start_lens[b] : a.start_len;
+  const int start = __builtin_amdgcn_readfirstlane(a.start_lens ? a.start_lens[b] : a.start_len);
   if (start < 0 || a.num_new < 1) return;
   if (x < 2 * g.nkv) {
     const AppendSpan sp(g, start, a.num_new);
     if (__builtin_expect(sp.D == 0, 1))  // first, and short: most calls fetch no other code
       append_rows<HD, false>(g, a, b, x >> 1, x & 1, wave, sp.r0, a.num_new, lane);
     else if (x & 1)
-      append_slice<HD, true, false>(g, a, b, x >> 1, wave, start, a.num_new, lane);
+      append_slice<HD, true, false>(g, a, b, x >> 1, wave, start, a.num_new, lane, [] {});
     else
-      append_slice<HD, false, false>(g, a, b, x >> 1, wave, start, a.num_new, lane);
+      append_slice<HD, false, false>(g, a, b, x >> 1, wave, start, a.num_new, lane, [] {});
     return;
   }
   const int it = (x - 2 * g.nkv) * WPB + wave;

@@ -1,0 +1,84 @@
+"""The decode of calls of few segments (at most one (sequence, kv head) per CU):
+a workgroup per chunk of a segment, folded in LDS and across workgroups.  Lengths
+lie around where a segment is cut (three units per wavefront), at the edges of
+groups and of the fp16 window, and where the fused step ages a group out of a
+cut segment; batches around where the call leaves this kernel and where its
+sequences fill more than one window of 64."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from jacq_amd import workloads as wl
+from oracle import oracle as o
+from tests.kivi_testlib import State, assert_close, to_torch
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+POOL = ("k_code", "k_scale", "k_zero", "v_code", "v_scale", "v_zero", "k_scr", "v_scr")
+
+
+def _bits(t):
+    t = t.detach().cpu()
+    return (t.view(torch.int16) if t.dtype == torch.float16 else t).numpy()
+
+
+def _check(nh, nkv, hd, page, R, lens, seed):
+    """A decode and two fused steps (the first ages a group out wherever a
+    length is R + 31 modulo 32), eager and replayed, against the oracle."""
+    from jacq_amd import kivi
+    w = wl.Workload("chunks", nh, nkv, hd, len(lens), 1, 1, page=page, residual=R, outliers=2,
+                    outlier_scale=9.0, seed=3)
+    st = State(w, lens=lens, extra_tokens=2, seed=seed)
+    st.build_oracle()
+    geo = kivi.KiviGeometry(nh, nkv, hd, page, 32, R, st.max_pages, st.num_pages)
+    cache = kivi.PagedKiviCache.from_tensors(geo, to_torch(st))
+    q = torch.from_numpy(st.q).view(torch.float16).cuda()
+    bt = torch.from_numpy(st.tables).cuda()
+    n = torch.from_numpy(st.lens.astype(np.int32)).cuda()
+    out = cache.decode(q, n, bt)
+    assert_close(out.cpu().numpy(), st.decode_ref(), "decode")
+    graph, again = torch.cuda.CUDAGraph(), torch.empty_like(out)
+    with torch.cuda.graph(graph):
+        cache.decode(q, n, bt, out=again)
+    for _ in range(3):  # the flags are clear after each replay
+        again.fill_(3.0)
+        graph.replay()
+        assert torch.equal(again.view(torch.int32), out.view(torch.int32))
+    cur = st.lens.copy()
+    for _ in range(2):
+        new = [torch.from_numpy(np.stack([h[b][cur[b]] for b in range(len(lens))])).view(
+            torch.float16).cuda() for h in (st.k_hist, st.v_hist)]
+        out = cache.write_decode(q, *new, torch.from_numpy((cur + 1).astype(np.int32)).cuda(), bt)
+        for b in range(len(lens)):
+            o.cache_write(st.cache, b, st.k_hist[b][cur[b]], st.v_hist[b][cur[b]], st.tables[b],
+                          int(cur[b]) + 1)
+        cur = cur + 1
+        torch.cuda.synchronize()
+        for name in POOL:
+            want = getattr(st.cache, name)
+            assert np.array_equal(_bits(getattr(cache, name)).view(want.dtype), want), name
+        assert_close(out.cpu().numpy(), st.decode_ref(cur), "fused step")
+
+
+@pytest.mark.parametrize("nh,nkv,hd,page,R", [(10, 2, 128, 16, 128), (32, 2, 128, 32, 64),
+                                              (7, 1, 64, 16, 32), (24, 2, 64, 32, 128)])
+def test_lengths_around_the_cut(nh, nkv, hd, page, R):
+    whole = 24 if hd == 128 and nh // nkv > 8 else 36  # units of a segment kept whole
+    groups = whole - 3 * (R // 32)
+    edge = R + 32 * groups  # this many units, and one token more starts a residual tile
+    _check(nh, nkv, hd, page, R, [edge - 1, edge, edge + 1, edge + 31, edge + 32, R + 31, R + 32,
+                                  R - 1, 31, 1, 2 * edge + 31, 12 * edge + 31], seed=nh)
+
+
+@pytest.mark.parametrize("batch,nkv", [(128, 2), (129, 2), (64, 4), (256, 1), (193, 1)])
+def test_batches_around_one_segment_per_cu(batch, nkv):
+    lens = [1 + (37 * i) % 190 for i in range(batch)]
+    lens[::7] = [63 + 32 * (i % 40) for i in range(len(lens[::7]))]
+    _check(2 * nkv, nkv, 64, 16, 32, lens, seed=batch)
+
+
+def test_one_long_sequence_among_short_ones():
+    lens = [20, 150, 9000, 159, 33, 700]
+    _check(40, 8, 128, 16, 128, lens, seed=5)
