@@ -18,8 +18,9 @@ layer raises ``NativeLibraryMissing``.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
-from dataclasses import dataclass
+from dataclasses import dataclass, fields
 
 import torch
 
@@ -441,6 +442,14 @@ class KiviGeometry:
         return Geometry(self.num_heads, self.num_kv_heads, self.head_dim, self.page_size,
                         self.group_size, self.residual, self.max_pages_per_seq, self.num_pages)
 
+    @functools.cached_property
+    def ref(self):
+        """The record by reference, made once: the fields never change."""
+        return ctypes.byref(self.c())
+
+    def __getstate__(self):  # copies and pickles carry the fields alone
+        return {f.name: getattr(self, f.name) for f in fields(self)}
+
     def check(self) -> None:
         g = self.c()
         if lib().jacq_kivi_check_geometry(ctypes.byref(g)) != 0:
@@ -449,6 +458,12 @@ class KiviGeometry:
     def max_seq_len(self) -> int:
         return ((self.max_pages_per_seq * self.page_size) // self.group_size) * self.group_size \
             + self.residual
+
+
+def _raw_stream(t: torch.Tensor) -> int:
+    """The current stream of the tensor's device, without a Stream object."""
+    index = t.get_device()
+    return torch._C._cuda_getCurrentRawStream(index) if index >= 0 else _stream(t.device).value
 
 
 class PagedKiviCache:
@@ -495,25 +510,61 @@ class PagedKiviCache:
         return (self.k_code, self.k_scale, self.k_zero, self.v_code, self.v_scale, self.v_zero,
                 self.k_scr, self.v_scr)
 
+    def _pool_ptrs(self):
+        return (self.k_code.data_ptr(), self.k_scale.data_ptr(), self.k_zero.data_ptr(),
+                self.v_code.data_ptr(), self.v_scale.data_ptr(), self.v_zero.data_ptr(),
+                self.k_scr.data_ptr(), self.v_scr.data_ptr())
+
+    # The checks of a call in one expression each: a decode of a small model takes
+    # the GPU about 10 us, and the named checks and argument objects took the host
+    # as long.  A call that fails one goes to the named checks, which say why.
+
+    def _fits(self, lens: torch.Tensor, block_tables: torch.Tensor) -> bool:
+        return (lens.shape == (self.batch,) and lens.dtype is torch.int32
+                and block_tables.shape == (self.batch, self.geo.max_pages_per_seq)
+                and block_tables.dtype is torch.int32 and block_tables.is_contiguous())
+
+    def _fits_query(self, q: torch.Tensor) -> bool:
+        g = self.geo
+        return (q.shape == (self.batch, g.num_heads, g.head_dim) and q.dtype is torch.float16
+                and q.is_contiguous())
+
+    def _check_tables(self, lens: torch.Tensor, block_tables: torch.Tensor) -> None:
+        check_shape(lens, (self.batch,), "SEQ_LENS")
+        _check(lens.dtype == torch.int32, "SEQ_LENS must be int32")
+        check_shape(block_tables, (self.batch, self.geo.max_pages_per_seq), "BLOCK_TABLES")
+        _check(block_tables.dtype == torch.int32 and block_tables.is_contiguous(),
+               "BLOCK_TABLES must be contiguous int32")
+
+    def _check_query(self, q: torch.Tensor) -> None:
+        check_shape(q, (self.batch, self.geo.num_heads, self.geo.head_dim), "Q")
+        _check(q.dtype == torch.float16 and q.is_contiguous(), "Q must be contiguous fp16")
+
     def append(self, new_k: torch.Tensor, new_v: torch.Tensor, block_tables: torch.Tensor,
                start_lens: torch.Tensor) -> None:
         """new_k/new_v [batch, num_new, NKV, HD] fp16; start_lens [batch] int32."""
         g = self.geo
-        _check(new_k.dim() == 4 and new_k.shape[0] == self.batch
-               and new_k.shape[2:] == (g.num_kv_heads, g.head_dim), "NEW_K shape mismatch")
-        _check(new_v.shape == new_k.shape, "NEW_V shape mismatch")
-        _check(new_k.dtype == torch.float16 and new_v.dtype == torch.float16, "NEW_K/V must be fp16")
-        _check(new_k.is_contiguous() and new_v.is_contiguous(), "NEW_K/V must be contiguous")
-        check_shape(block_tables, (self.batch, g.max_pages_per_seq), "BLOCK_TABLES")
-        _check(block_tables.dtype == torch.int32 and block_tables.is_contiguous(),
-               "BLOCK_TABLES must be contiguous int32")
-        check_shape(start_lens, (self.batch,), "START_LENS")
-        _check(start_lens.dtype == torch.int32, "START_LENS must be int32")
-        geo = g.c()
-        rc = lib().jacq_kivi_cache_append(ctypes.byref(geo), *[_ptr(t) for t in self.pool()],
-                                          _ptr(new_k), _ptr(new_v), _ptr(block_tables),
-                                          _ptr(start_lens), int(new_k.shape[1]), self.batch,
-                                          _stream(new_k.device))
+        shape = new_k.shape
+        if not (len(shape) == 4 and shape[0] == self.batch
+                and shape[2] == g.num_kv_heads and shape[3] == g.head_dim
+                and new_v.shape == shape and new_k.dtype is torch.float16
+                and new_v.dtype is torch.float16 and new_k.is_contiguous()
+                and new_v.is_contiguous() and self._fits(start_lens, block_tables)):
+            _check(new_k.dim() == 4 and new_k.shape[0] == self.batch
+                   and new_k.shape[2:] == (g.num_kv_heads, g.head_dim), "NEW_K shape mismatch")
+            _check(new_v.shape == new_k.shape, "NEW_V shape mismatch")
+            _check(new_k.dtype == torch.float16 and new_v.dtype == torch.float16,
+                   "NEW_K/V must be fp16")
+            _check(new_k.is_contiguous() and new_v.is_contiguous(), "NEW_K/V must be contiguous")
+            check_shape(block_tables, (self.batch, g.max_pages_per_seq), "BLOCK_TABLES")
+            _check(block_tables.dtype == torch.int32 and block_tables.is_contiguous(),
+                   "BLOCK_TABLES must be contiguous int32")
+            check_shape(start_lens, (self.batch,), "START_LENS")
+            _check(start_lens.dtype == torch.int32, "START_LENS must be int32")
+        rc = lib().jacq_kivi_cache_append(g.ref, *self._pool_ptrs(), new_k.data_ptr(),
+                                          new_v.data_ptr(), block_tables.data_ptr(),
+                                          start_lens.data_ptr(), shape[1], self.batch,
+                                          _raw_stream(new_k))
         if rc != 0:
             raise KiviLaunchError(last_error())
 
@@ -522,21 +573,17 @@ class PagedKiviCache:
                ) -> torch.Tensor:
         """q [batch, NH, HD] fp16 -> O [batch, NH, HD] fp32."""
         g = self.geo
-        check_shape(q, (self.batch, g.num_heads, g.head_dim), "Q")
-        _check(q.dtype == torch.float16 and q.is_contiguous(), "Q must be contiguous fp16")
-        check_shape(seq_lens, (self.batch,), "SEQ_LENS")
-        _check(seq_lens.dtype == torch.int32, "SEQ_LENS must be int32")
-        check_shape(block_tables, (self.batch, g.max_pages_per_seq), "BLOCK_TABLES")
-        _check(block_tables.dtype == torch.int32 and block_tables.is_contiguous(),
-               "BLOCK_TABLES must be contiguous int32")
+        if not (self._fits_query(q) and self._fits(seq_lens, block_tables)):
+            self._check_query(q)
+            self._check_tables(seq_lens, block_tables)
         if out is None:
             out = torch.empty((self.batch, g.num_heads, g.head_dim), dtype=torch.float32,
                               device=q.device)
-        geo = g.c()
-        ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-        rc = lib().jacq_kivi_decode(ctypes.byref(geo), _ptr(q), _ptr(seq_lens), _ptr(block_tables),
-                                    *[_ptr(t) for t in self.pool()], self.batch, _ptr(out),
-                                    _ptr(workspace), ws_bytes, _stream(q.device))
+        ws, ws_bytes = ((0, 0) if workspace is None else
+                        (workspace.data_ptr(), workspace.numel() * workspace.element_size()))
+        rc = lib().jacq_kivi_decode(g.ref, q.data_ptr(), seq_lens.data_ptr(),
+                                    block_tables.data_ptr(), *self._pool_ptrs(), self.batch,
+                                    out.data_ptr(), ws, ws_bytes, _raw_stream(q))
         if rc != 0:
             _raise(rc)
         return out
@@ -549,25 +596,26 @@ class PagedKiviCache:
         [batch, NKV, HD] fp16 at position seq_lens - 1, then decode q
         [batch, NH, HD] over the new state -> O [batch, NH, HD] fp32."""
         g = self.geo
-        check_shape(q, (self.batch, g.num_heads, g.head_dim), "Q")
-        _check(q.dtype == torch.float16 and q.is_contiguous(), "Q must be contiguous fp16")
-        for t, name in ((new_k, "NEW_K"), (new_v, "NEW_V")):
-            check_shape(t, (self.batch, g.num_kv_heads, g.head_dim), name)
-            _check(t.dtype == torch.float16 and t.is_contiguous(), name + " must be contiguous fp16")
-        check_shape(seq_lens, (self.batch,), "SEQ_LENS")
-        _check(seq_lens.dtype == torch.int32, "SEQ_LENS must be int32")
-        check_shape(block_tables, (self.batch, g.max_pages_per_seq), "BLOCK_TABLES")
-        _check(block_tables.dtype == torch.int32 and block_tables.is_contiguous(),
-               "BLOCK_TABLES must be contiguous int32")
+        token = (self.batch, g.num_kv_heads, g.head_dim)
+        if not (self._fits_query(q) and new_k.shape == token and new_v.shape == token
+                and new_k.dtype is torch.float16 and new_v.dtype is torch.float16
+                and new_k.is_contiguous() and new_v.is_contiguous()
+                and self._fits(seq_lens, block_tables)):
+            self._check_query(q)
+            for t, name in ((new_k, "NEW_K"), (new_v, "NEW_V")):
+                check_shape(t, token, name)
+                _check(t.dtype == torch.float16 and t.is_contiguous(),
+                       name + " must be contiguous fp16")
+            self._check_tables(seq_lens, block_tables)
         if out is None:
             out = torch.empty((self.batch, g.num_heads, g.head_dim), dtype=torch.float32,
                               device=q.device)
-        geo = g.c()
-        ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
-        rc = lib().jacq_kivi_write_decode(ctypes.byref(geo), _ptr(q), _ptr(new_k), _ptr(new_v),
-                                          _ptr(seq_lens), _ptr(block_tables),
-                                          *[_ptr(t) for t in self.pool()], self.batch, _ptr(out),
-                                          _ptr(workspace), ws_bytes, _stream(q.device))
+        ws, ws_bytes = ((0, 0) if workspace is None else
+                        (workspace.data_ptr(), workspace.numel() * workspace.element_size()))
+        rc = lib().jacq_kivi_write_decode(g.ref, q.data_ptr(), new_k.data_ptr(),
+                                          new_v.data_ptr(), seq_lens.data_ptr(),
+                                          block_tables.data_ptr(), *self._pool_ptrs(), self.batch,
+                                          out.data_ptr(), ws, ws_bytes, _raw_stream(q))
         if rc != 0:
             _raise(rc)
         return out
@@ -587,12 +635,12 @@ class PagedKiviCache:
                "RETAINED_BLOCK_TABLE holds fewer than NUM_RETAINED_PAGES entries")
         if out is None:
             out = torch.empty((g.num_heads, g.head_dim), dtype=torch.float32, device=q.device)
-        geo = g.c()
-        ws_bytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+        ws, ws_bytes = ((0, 0) if workspace is None else
+                        (workspace.data_ptr(), workspace.numel() * workspace.element_size()))
         rc = lib().jacq_kivi_decode_sparse_retained(
-            ctypes.byref(geo), _ptr(q), int(seq_len), _ptr(retained_table),
-            int(num_retained_pages), *[_ptr(t) for t in self.pool()], _ptr(out),
-            _ptr(workspace), ws_bytes, _stream(q.device))
+            g.ref, q.data_ptr(), int(seq_len), retained_table.data_ptr(),
+            int(num_retained_pages), *self._pool_ptrs(), out.data_ptr(), ws, ws_bytes,
+            _raw_stream(q))
         if rc != 0:
             _raise(rc)
         return out
