@@ -1849,8 +1849,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
 
 // ---- calls of few segments: one workgroup per chunk of a segment ----
 //
-// With at most one (sequence, kv head) segment per CU the stream above cuts
-// every segment among many wavefronts, and the merge of their partials, two or
+// With few (sequence, kv head) segments the stream above cuts every segment
+// among many wavefronts, and the merge of their partials, two or
 // eight per memory round, outlasts the decode: 65 pieces per segment in a
 // 16k-token sequence at 8 kv heads took 36 of 52 us.  Here a workgroup of nw
 // wavefronts takes a chunk of one segment: its wavefronts decode nw equal runs of the
@@ -1884,7 +1884,7 @@ __device__ inline int chunk_count(int units, int cu, int whole) {
   return units <= whole ? 1 : (units + cu - 1) / cu;
 }
 
-// Sequences a call of the chunk kernel may hold: at most one segment per CU.
+// Sequences a call of the chunk kernel may hold.
 constexpr int kChunkWindows = 4;  // of 64 sequences, one per lane
 
 // Units per chunk of a whole call: the fewest that make no more chunks than
@@ -2269,14 +2269,26 @@ static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream
     launch_one<HD, P, false>(g, a, stream, start, stop);
 }
 
-// Calls of at most one segment per CU go to the chunk kernel, and all of the v1
-// symbols', whose queries must decode to the same bits alone and together.
-//  - Whole calls take the largest workgroup a CU holds (twelve wavefronts, eight of
-//    the HD 128 kernel for G > 8): the fold in LDS costs 1 us whatever their number,
-//    a cut between workgroups 4 us.  So a segment of up to three units per wavefront
-//    (3 us) stays whole, and a longer one is cut down to one unit per
-//    wavefront where workgroups are free (2 and 3 units were 1 to 2 us slower for
-//    one 16k-token sequence and for 16 of 2048 tokens).
+// To the chunk kernel go all calls of the v1 symbols, whose queries must decode
+// to the same bits alone and together, and calls
+//  - of at most three segments per eight CUs: 12 sequences of 100 to 32000 tokens (40 / 8
+//    heads) 84.7 us in the stream, 56.5 here, 4 of them 113.5 / 28.8, 48 at 14 / 2
+//    heads, HD 64, 50.0 / 42.5.  With more there is too little room to cut the
+//    long ones: 80 of those at HD 64 63.9 / 74.7, 32 of 1000 to 32000 at HD 128 139 / 184;
+//  - of at most one segment per four wavefronts of the device, if the table bounds their
+//    work by 24 units per resident wavefront (12 at HD 64, whose stream folds eight
+//    partials a round: 128 of 100 to 8000 36.4 / 42.5): 64 sequences of 200 to 400 tokens
+//    27.3 / 23.0, of 1000 to 2000 with a write 50.3 / 48.0, of 2000 to 4000 67.4 /
+//    66.7; but of 1000 to 8000 86.2 / 91.1 and of 1024 to 16384 149.6 / 164.9, where
+//    the stream's equal runs balance better than whole chunks.
+// How they are cut:
+//  - Calls of at most one segment per CU take the largest workgroup a CU holds (twelve
+//    wavefronts, eight of the HD 128 kernel for G > 8): the fold in LDS costs 1 us
+//    whatever their number, a cut between workgroups 4 us.  Calls of more take
+//    four wavefronts, three or two workgroups to a CU.  A segment of up to three
+//    units per wavefront (3 us) stays whole, and a longer one is cut down to one
+//    unit per wavefront where workgroups are free (2 and 3 units were 1 to 2 us
+//    slower for one 16k-token sequence and for 16 of 2048 tokens).
 //  - The v1 symbols take four wavefronts and 16 units: one 2900-token query is
 //    faster with fewer units (8: 15.8 us against 17.0 with its write; 32: 20.3),
 //    31 causal ones with more (47 us; 8: 65, 32: 41).
@@ -2284,13 +2296,16 @@ ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_
   ChunkPlan p{};
   const int most = g.hd == 128 && g.gqa > 8 ? 8 : 12;
   const int64_t segs = (int64_t)batch * g.nkv;
-  if (!per_query && (segs > cus || batch > 64 * kChunkWindows)) return p;
-  p.waves = per_query ? 4 : most;
-  p.units = per_query ? 16 : most;
-  p.whole = per_query ? 0 : 3 * most;
   const int64_t tiles = std::max<int64_t>(1, (max_tokens + kGroup - 1) / kGroup);
   // a segment's units at most: R / 32 + 1 of its tiles are residual
   const int64_t units = tiles + (kResidualUnits - 1) * (g.residual / kGroup + 1);
+  const bool few = 8 * segs <= 3ll * cus;
+  const bool small = segs <= (int64_t)cus * (most / 4) &&
+                     segs * units <= (g.hd == 64 ? 12ll : 24ll) * most * cus;
+  if (!per_query && ((!few && !small) || batch > 64 * kChunkWindows)) return p;
+  p.waves = per_query || segs > cus ? 4 : most;
+  p.units = per_query ? 16 : p.waves;
+  p.whole = per_query ? 0 : 3 * p.waves;
   const int64_t per_segment = units <= p.whole ? 1 : (units + p.units - 1) / p.units;
   if (per_query) p.per_query = (int)(g.nkv * per_segment);
   p.slots = cus * (most / p.waves);

@@ -1,5 +1,5 @@
-"""The decode of calls of few segments (at most one (sequence, kv head) per CU):
-a workgroup per chunk of a segment, folded in LDS and across workgroups.  Lengths
+"""The decode of calls of few or short segments ((sequence, kv head) pairs): a
+workgroup per chunk of a segment, folded in LDS and across workgroups.  Lengths
 lie around where a segment is cut (three units per wavefront), at the edges of
 groups and of the fp16 window, and where the fused step ages a group out of a
 cut segment; batches around where the call leaves this kernel and where its
@@ -72,8 +72,9 @@ def test_lengths_around_the_cut(nh, nkv, hd, page, R):
                                   R - 1, 31, 1, 2 * edge + 31, 12 * edge + 31], seed=nh)
 
 
-@pytest.mark.parametrize("batch,nkv", [(128, 2), (129, 2), (64, 4), (256, 1), (193, 1)])
-def test_batches_around_one_segment_per_cu(batch, nkv):
+@pytest.mark.parametrize("batch,nkv", [(128, 2), (129, 2), (64, 4), (256, 1), (257, 1), (193, 1),
+                                       (96, 8), (97, 8)])
+def test_batches_around_the_rules_segment_counts(batch, nkv):
     lens = [1 + (37 * i) % 190 for i in range(batch)]
     lens[::7] = [63 + 32 * (i % 40) for i in range(len(lens[::7]))]
     _check(2 * nkv, nkv, 64, 16, 32, lens, seed=batch)
