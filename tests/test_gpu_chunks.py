@@ -83,3 +83,25 @@ def test_batches_around_the_rules_segment_counts(batch, nkv):
 def test_one_long_sequence_among_short_ones():
     lens = [20, 150, 9000, 159, 33, 700]
     _check(40, 8, 128, 16, 128, lens, seed=5)
+
+
+def test_v1_queries_of_two_launches_equal_single():
+    """160 causal queries of one 4096-token sequence need two launches of a v1
+    workspace region; each equals its own jac_launch bit for bit."""
+    from jacq_amd import kivi
+    w = wl.Workload("v1", 40, 8, 128, 1, 4096, 4096, page=32, residual=128, outliers=8, seed=11)
+    st = State(w, lens=[4096], seed=8)
+    st.build_oracle()
+    g = to_torch(st)
+    bt = torch.from_numpy(st.tables[0]).cuda()
+    pool = [g[n] for n in POOL[:6]] + [g["k_scr"][0], g["v_scr"][0]]
+    seq = np.arange(4096 - 159, 4097).astype(np.int32)
+    seq[:4] = [1, 129, 160, 1000]
+    q = torch.from_numpy(np.random.default_rng(3).standard_normal((160, 40, 128)).astype(
+        np.float16)).cuda()
+    out = torch.empty((160, 40, 128), dtype=torch.float32, device="cuda")
+    kivi.kivi_decode_batched_dsl(q, torch.from_numpy(seq).cuda(), bt, *pool, 160, out)
+    one = torch.empty((40, 128), dtype=torch.float32, device="cuda")
+    for i in list(range(0, 160, 13)) + [1, 2, 3, 88, 89, 90, 159]:
+        kivi.kivi_decode_dsl(q[i].contiguous(), bt, *pool, int(seq[i]), one)
+        assert torch.equal(one.view(torch.int32), out[i].view(torch.int32)), i
