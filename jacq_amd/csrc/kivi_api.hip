@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <initializer_list>
+#include <iterator>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -639,6 +640,16 @@ int64_t jacq_kivi_test_device_allocations(void) {
 
 void jacq_kivi_test_force_merge_timeout(uint32_t microseconds) {
   jacq::set_test_merge_timeout_us(microseconds);
+}
+
+// Test hook outside the ABI (no declaration in jacq_kivi.h): how a whole-call or
+// per-query decode on a device of `cus` CUs would be cut; out[0] == 0: the stream kernel.
+void jacq_kivi_test_plan_decode(const jacq_kivi_geometry* geo, int32_t batch, int64_t max_tokens,
+                                int32_t per_query, int32_t cus, int32_t* out) {
+  const jacq::ChunkPlan p =
+      jacq::plan_chunks(make_geo(*geo), batch, max_tokens, per_query != 0, cus);
+  const int32_t v[] = {p.waves, p.grid, p.slots, p.units, p.whole};
+  std::copy(std::begin(v), std::end(v), out);
 }
 
 int64_t jacq_kivi_max_seq_len(const jacq_kivi_geometry* geo) {

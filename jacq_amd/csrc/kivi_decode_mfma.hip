@@ -2270,17 +2270,30 @@ static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream
 }
 
 // To the chunk kernel go all calls of the v1 symbols, whose queries must decode
-// to the same bits alone and together, and calls
-//  - of at most three segments per eight CUs: 12 sequences of 100 to 32000 tokens (40 / 8
-//    heads) 84.7 us in the stream, 56.5 here, 4 of them 113.5 / 28.8, 48 at 14 / 2
-//    heads, HD 64, 50.0 / 42.5.  With more there is too little room to cut the
-//    long ones: 80 of those at HD 64 63.9 / 74.7, 32 of 1000 to 32000 at HD 128 139 / 184;
-//  - of at most one segment per four wavefronts of the device, if the table bounds their
-//    work by 24 units per resident wavefront (12 at HD 64, whose stream folds eight
-//    partials a round: 128 of 100 to 8000 36.4 / 42.5): 64 sequences of 200 to 400 tokens
-//    27.3 / 23.0, of 1000 to 2000 with a write 50.3 / 48.0, of 2000 to 4000 67.4 /
-//    66.7; but of 1000 to 8000 86.2 / 91.1 and of 1024 to 16384 149.6 / 164.9, where
-//    the stream's equal runs balance better than whole chunks.
+// to the same bits alone and together, and of the others those that no mix of lengths
+// makes slower here than in the stream.  The host knows the S segments and a bound U on
+// a segment's units (from the block table's width), not the lengths.  Where W workgroups
+// are resident, a long segment is sure of C = W / S of them, and with just over
+// (W - S) / C long segments among short ones it gets no more while S / W of the chip
+// idles: the longest run is then longer than the stream's equal ones by U / C units per
+// workgroup, times S / W.  What the chunk kernel saves is the stream's merge, a fixed
+// time.  So the bound is on S U / C per resident wavefront (`share`).  Stream / chunk in us
+// where the two meet, for the worst mix found:
+//  - HD 128, G <= 8, 12 units: 17 sequences (8 kv heads), 16 of them of 8352 tokens, 55.6 /
+//    57.3; 32, one of 4288, 35.1 / 35.3.  Equal lengths: 17 of 4000 tokens 42.7 / 34.3,
+//    of 16000 (beyond the bound) 84.0 / 102.7.  In workgroups of four
+//    wavefronts 5: 72 sequences, 25 of 352 tokens (4 units), 24.8 / 22.7, 25 of 704 (6
+//    units) 26.5 / 28.7.
+//  - HD 128, G > 8, whose stream folds one partial a round, 18: 44 sequences (2 kv
+//    heads), 43 of 26464 tokens, 107.1 / 98.5, of 35424 (24 units) 124.0 / 125.9.  In
+//    workgroups of four wavefronts 15: 132, 125 of 3392 tokens, 58.2 / 57.0, of 4128
+//    (18 units) 62.6 / 65.8.
+//  - HD 64, whose stream folds eight partials a round, 5: 44 (2 kv heads), 43 of 13056
+//    tokens (6 units), 41.8 / 40.6, of 17536 (8 units) 47.6 / 50.3; 3 where no segment is
+//    sure of a cut (C = 1): 96, 33 of 1216 tokens, 18.5 / 17.9, of 1728 (4 units) 19.3 /
+//    19.9; in workgroups of four wavefronts none that may be cut (132 of 300 tokens 17.5 / 18.0).
+// A call under a wide table may so take the stream where the same lengths under a tight
+// one come here.
 // How they are cut:
 //  - Calls of at most one segment per CU take the largest workgroup a CU holds (twelve
 //    wavefronts, eight of the HD 128 kernel for G > 8): the fold in LDS costs 1 us
@@ -2294,21 +2307,28 @@ static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream
 //    31 causal ones with more (47 us; 8: 65, 32: 41).
 ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_query, int cus) {
   ChunkPlan p{};
-  const int most = g.hd == 128 && g.gqa > 8 ? 8 : 12;
+  const bool wide = g.hd == 128 && g.gqa > 8;
+  const int most = wide ? 8 : 12;
   const int64_t segs = (int64_t)batch * g.nkv;
   const int64_t tiles = std::max<int64_t>(1, (max_tokens + kGroup - 1) / kGroup);
   // a segment's units at most: R / 32 + 1 of its tiles are residual
   const int64_t units = tiles + (kResidualUnits - 1) * (g.residual / kGroup + 1);
-  const bool few = 8 * segs <= 3ll * cus;
-  const bool small = segs <= (int64_t)cus * (most / 4) &&
-                     segs * units <= (g.hd == 64 ? 12ll : 24ll) * most * cus;
-  if (!per_query && ((!few && !small) || batch > 64 * kChunkWindows)) return p;
-  p.waves = per_query || segs > cus ? 4 : most;
+  const int waves = per_query || segs > cus ? 4 : most;
+  const int64_t slots = (int64_t)cus * (most / waves);
+  const int whole = per_query ? 0 : 3 * waves;
+  if (!per_query) {
+    if (segs > slots || batch > 64 * kChunkWindows) return p;
+    const int64_t cuts = slots / segs;
+    const int64_t share = segs > cus ? (g.hd == 64 ? 0 : wide ? 15 : 5)
+                                     : (g.hd == 64 ? (cuts > 1 ? 5 : 3) : wide ? 18 : 12);
+    if (units > whole && segs * units > share * cuts * most * cus) return p;
+  }
+  p.waves = waves;
   p.units = per_query ? 16 : p.waves;
-  p.whole = per_query ? 0 : 3 * p.waves;
+  p.whole = whole;
   const int64_t per_segment = units <= p.whole ? 1 : (units + p.units - 1) / p.units;
   if (per_query) p.per_query = (int)(g.nkv * per_segment);
-  p.slots = cus * (most / p.waves);
+  p.slots = (int)slots;
   p.grid = (int)std::min<int64_t>(segs * per_segment, p.slots);
   return p;
 }
