@@ -652,6 +652,10 @@ void jacq_kivi_test_plan_decode(const jacq_kivi_geometry* geo, int32_t batch, in
   std::copy(std::begin(v), std::end(v), out);
 }
 
+// Test hook outside the ABI: while on, whole-call decodes of the calling thread take the
+// stream kernel whatever their size (the v1 symbols stay with the chunk kernel).
+void jacq_kivi_test_force_stream(int32_t on) { jacq::set_test_force_stream(on != 0); }
+
 int64_t jacq_kivi_max_seq_len(const jacq_kivi_geometry* geo) {
   if (check_geometry(geo) != JACQ_KIVI_OK) return -1;
   return max_seq_len(*geo);

@@ -2305,8 +2305,12 @@ static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream
 //  - The v1 symbols take four wavefronts and 16 units: one 2900-token query is
 //    faster with fewer units (8: 15.8 us against 17.0 with its write; 32: 20.3),
 //    31 causal ones with more (47 us; 8: 65, 32: 41).
+static thread_local bool t_test_stream = false;
+void set_test_force_stream(bool on) { t_test_stream = on; }
+
 ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_query, int cus) {
   ChunkPlan p{};
+  if (t_test_stream && !per_query) return p;
   const bool wide = g.hd == 128 && g.gqa > 8;
   const int most = wide ? 8 : 12;
   const int64_t segs = (int64_t)batch * g.nkv;

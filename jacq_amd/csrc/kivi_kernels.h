@@ -118,6 +118,8 @@ struct ChunkPlan {
   int per_query;  // per-query split: chunks of a query at most (all kv heads)
 };
 ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_query, int cus);
+// Test-only: while on, the calling thread's whole-call decodes take the stream kernel.
+void set_test_force_stream(bool on);
 // wavefronts the matrix-core decode launches on a device with `cus` CUs:
 // as many as are resident at once
 int decode_stream_waves(const KiviGeo& g, int cus);
