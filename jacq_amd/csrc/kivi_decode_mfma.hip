@@ -816,10 +816,13 @@ __device__ inline int64_t stream_units(const KiviGeo& g, const DecodeArgs& a, in
 // kMinUnitsPerWave units each, so that small batches spread over enough
 // wavefronts to hide the per-group latency chain without cutting every
 // segment into pieces the merge must fold (4: TinyLlama 17.9 -> 15.6 us,
-// Qwen0.5B 19.6 -> 18.5 us against 8; 2 was slower at Qwen0.5B).
-constexpr int kMinUnitsPerWave = 4;
+// Qwen0.5B 19.6 -> 18.5 us against 8; 2 was slower at Qwen0.5B).  A stream of
+// fewer than kTinyStream units (short sequences under a wide table) takes 2 per
+// wavefront (0.9 us faster at TinyLlama's 72; 1 was slower).
+constexpr int kMinUnitsPerWave = 4, kTinyStream = 256;
 __device__ inline int64_t stream_waves(int64_t units, int grid) {
-  int64_t w = (units + kMinUnitsPerWave - 1) / kMinUnitsPerWave;
+  const int per = units < kTinyStream ? 2 : kMinUnitsPerWave;
+  int64_t w = (units + per - 1) / per;
   if (w < 1) w = 1;
   return w < grid ? w : grid;
 }

@@ -74,3 +74,24 @@ def test_more_than_one_window_of_sequences(nh, nkv, hd, page, R):
     out, of which every third ages a group out at the first step."""
     lens = [R + 31 + 32 * (i % 9) if i % 3 == 0 else 1 + (53 * i) % 400 for i in range(67)]
     chunks._check(nh, nkv, hd, page, R, lens, seed=nh)
+
+
+@pytest.mark.parametrize("lens,most", [([40, 130, 3], 2), ([3000, 40, 2000], 4)])
+def test_units_per_wavefront(kivi, lens, most):  # noqa: F811
+    """A stream of fewer than 256 units is cut into runs of two, any other short of the
+    device's wavefronts into runs of four."""
+    w = wl.WORKLOADS["tinyllama"].scaled(batch=len(lens), ctx_lo=32)
+    st = State(w, lens=lens, seed=6)
+    st.build_oracle()
+    geo = kivi.KiviGeometry(w.nh, w.nkv, w.hd, w.page, 32, w.residual, st.max_pages, st.num_pages)
+    cache = kivi.PagedKiviCache.from_tensors(geo, to_torch(st))
+    stamps = torch.zeros((8192, 4), dtype=torch.int64, device="cuda")
+    assert kivi.lib().jacq_kivi_profile_wave_stamps(kivi._ptr(stamps), 8192) == 0
+    try:
+        cache.decode(torch.from_numpy(st.q).view(torch.float16).cuda(),
+                     torch.from_numpy(st.lens.astype(np.int32)).cuda(),
+                     torch.from_numpy(st.tables).cuda())
+        torch.cuda.synchronize()
+    finally:
+        assert kivi.lib().jacq_kivi_profile_wave_stamps(None, 0) == 0
+    assert int((stamps[:, 3] & 0xFFFFFFFF).max()) == most
