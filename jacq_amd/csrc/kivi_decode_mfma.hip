@@ -1018,19 +1018,24 @@ __device__ inline void st_agent(void* p, float lo, float hi) {
 __device__ inline void st_agent4(float* p, floatx4 v) {
   asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
-// 16-byte agent-scope load; the caller waits with an explicit vmcnt(0) and
-// then passes the value through keep() so no use moves above the wait
-__device__ inline floatx4 ld_agent4(const float* p) {
-  floatx4 v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
-  return v;
+// Agent-scope loads of a partial through a buffer descriptor over `bytes` bytes from a
+// wave-uniform base: beyond them (outputs past G * HD, no partial) a load reads zeros,
+// so none is under a branch.  Builtins, not asm: the compiler tracks what is in flight.
+__device__ inline __amdgpu_buffer_rsrc_t partial_rsrc(const float* p, int bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, bytes, 0x00020000);
 }
-__device__ inline void keep(floatx4& v) { asm volatile("" : "+v"(v)); }
-// Device-scope (sc1) store of one to eight bytes: the fused step's writer
-// stores what decode wavefronts of the same launch, on any XCD, read next.
-template <typename T>
-__device__ inline void st_dev(T* p, T v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+constexpr int kAgentScope = 16;  // sc1, what an agent-scope atomic load carries
+__device__ inline floatx4 ld_agent4(__amdgpu_buffer_rsrc_t r, int offset) {
+  return __builtin_bit_cast(floatx4,
+                            __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, kAgentScope));
+}
+__device__ inline uint64_t ld_agent2(__amdgpu_buffer_rsrc_t r, int offset) {
+  return __builtin_bit_cast(uint64_t,
+                            __builtin_amdgcn_raw_buffer_load_b64(r, offset, 0, kAgentScope));
+}
+__device__ inline float mul_rounded(float a, float b) {
+#pragma clang fp contract(off)
+  return a * b;
 }
 __device__ inline float lo_f(uint64_t v) { return __uint_as_float((uint32_t)v); }
 __device__ inline float hi_f(uint64_t v) { return __uint_as_float((uint32_t)(v >> 32)); }
@@ -1166,25 +1171,25 @@ __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const K
           ++rounds_after;
           uint64_t ml[U][K];
           floatx4 vv[U][K];
+          asm volatile("" ::: "memory");  // no load moves above its partial's flag
 #pragma unroll
           for (int u = 0; u < U; ++u) {
+            const bool have = slot[u] >= 0;
+            const auto rm = partial_rsrc(a.ws_ml + max(slot[u], (int64_t)0) * G * 2, have ? 8 * G : 0);
+            const auto rv =
+                partial_rsrc(a.ws_acc + max(slot[u], (int64_t)0) * G * HD, have ? 16 * n4 : 0);
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-              ml[u][k] = 0xff800000u;  // (m, l) = (-inf, 0): folded with weight 0
-              vv[u][k] = floatx4{0.f, 0.f, 0.f, 0.f};
-              if (slot[u] >= 0 && on[k]) {
-                const int64_t p = slot[u] * G + gi[k];
-                ml[u][k] = ld_agent(a.ws_ml + 2 * p);
-                vv[u][k] = ld_agent4(a.ws_acc + p * HD + d[k]);
-              }
+              ml[u][k] = ld_agent2(rm, 8 * gi[k]);
+              vv[u][k] = ld_agent4(rv, 16 * (lane + 64 * k));
             }
           }
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
+          for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int k = 0; k < K; ++k) keep(vv[u][k]);
-          }
+            for (int k = 0; k < K; ++k)
+              if (slot[u] < 0) ml[u][k] = 0xff800000u;  // (m, l) = (-inf, 0): folded with weight 0
           // read: clear the flags, so the next launch starts from zero even
           // when it carries the same epoch (a replayed graph does)
           if (consumed & bit)
@@ -1198,9 +1203,13 @@ __device__ __attribute__((always_inline)) inline uint64_t merge_segments(const K
               const float mn = fmaxf(M[k], m);
               const float fo = __builtin_amdgcn_exp2f(M[k] - mn);
               const float fn = __builtin_amdgcn_exp2f(m - mn);
-              const floatx4 v = vv[u][k];
-              acc[k] = acc[k] * fo + v * fn;
-              Lsum[k] = Lsum[k] * fo + l * fn;
+              // the products' roundings written out: which of the U steps takes a
+              // partial depends on timing, and left to itself the compiler may
+              // fuse one step's other product
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+                acc[k][i] = __builtin_fmaf(acc[k][i], fo, mul_rounded(vv[u][k][i], fn));
+              Lsum[k] = __builtin_fmaf(Lsum[k], fo, mul_rounded(l, fn));
               M[k] = mn;
             }
           }
@@ -2202,12 +2211,9 @@ __global__ __launch_bounds__(64 * (coop_max_waves<HD, PACK>())) void kivi_decode
 #pragma unroll
             for (int k = 0; k < N; ++k) {  // past the last: the last again, with weight 0
               const int64_t at = (int64_t)(x - ci + min(k0 + k, cnt - 1)) * G;
-              pml[k] = ld_agent(a.ws_ml + 2 * (at + gi));
-              pv[k] = ld_agent4(a.ws_acc + at * HD + 4 * e);
+              pml[k] = ld_agent2(partial_rsrc(a.ws_ml + 2 * at, 8 * G), 8 * gi);
+              pv[k] = ld_agent4(partial_rsrc(a.ws_acc + at * HD, 16 * n4), 16 * e);
             }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int k = 0; k < N; ++k) keep(pv[k]);
 #pragma unroll
             for (int k = 0; k < N; ++k) {
               const float m = lo_f(pml[k]);
