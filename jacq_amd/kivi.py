@@ -18,9 +18,8 @@ layer raises ``NativeLibraryMissing``.
 from __future__ import annotations
 
 import ctypes
-import functools
 import os
-from dataclasses import dataclass, fields
+from dataclasses import dataclass
 
 import torch
 
@@ -419,8 +418,14 @@ def plan_batched_write(start_seq_len: int, num_new_tokens: int, residual: int = 
 # runtime-geometry surface
 # ---------------------------------------------------------------------------
 
+class _WithRecord:
+    """A place for the argument record outside the geometry's own attributes, which
+    vars(), copies and pickles show."""
+    __slots__ = ("_ref",)
+
+
 @dataclass(frozen=True)
-class KiviGeometry:
+class KiviGeometry(_WithRecord):
     num_heads: int
     num_kv_heads: int
     head_dim: int
@@ -442,13 +447,17 @@ class KiviGeometry:
         return Geometry(self.num_heads, self.num_kv_heads, self.head_dim, self.page_size,
                         self.group_size, self.residual, self.max_pages_per_seq, self.num_pages)
 
-    @functools.cached_property
+    @property
     def ref(self):
         """The record by reference, made once: the fields never change."""
-        return ctypes.byref(self.c())
+        try:
+            return self._ref
+        except AttributeError:
+            object.__setattr__(self, "_ref", ctypes.byref(self.c()))
+            return self._ref
 
-    def __getstate__(self):  # copies and pickles carry the fields alone
-        return {f.name: getattr(self, f.name) for f in fields(self)}
+    def __getstate__(self):  # copies and pickles carry the attributes, not the record
+        return dict(vars(self))
 
     def check(self) -> None:
         g = self.c()

@@ -444,3 +444,19 @@ def test_build_spill_guard_parses_resource_remarks():
     assert stream == {"vgprs": 161, "scratch": 12, "occupancy": 3}
     append = [v for k, v in r.items() if "kivi_append_kernel" in k][0]
     assert append["scratch"] == 0
+
+
+def test_geometry_shows_its_fields_alone():
+    """The argument record that a call leaves with a geometry is no attribute of it."""
+    import copy
+    import dataclasses
+    import pickle
+    geo = kivi.KiviGeometry(14, 2, 64, max_pages_per_seq=7, num_pages=9)
+    fields = dataclasses.asdict(geo)
+    assert geo.ref is geo.ref
+    assert vars(geo) == fields and kivi.KiviGeometry(**vars(geo)) == geo
+    for other in (copy.copy(geo), copy.deepcopy(geo), pickle.loads(pickle.dumps(geo)),
+                  dataclasses.replace(geo)):
+        assert other == geo and vars(other) == fields and other.ref is not geo.ref
+    with pytest.raises(dataclasses.FrozenInstanceError):
+        geo.num_pages = 1
