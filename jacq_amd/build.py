@@ -45,7 +45,7 @@ def hipcc() -> str:
 
 # Kernels that must not spill: a spill makes the kernel need scratch memory,
 # which cost the decode about 17 us (13%) when a 12-byte spill crept in.
-NO_SCRATCH = ("kivi_decode_stream_kernel", "kivi_append_kernel")
+NO_SCRATCH = ("kivi_decode_stream_kernel", "kivi_decode_chunk_kernel", "kivi_append_kernel")
 
 
 def kernel_resources(remarks: str) -> dict:

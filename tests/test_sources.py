@@ -42,3 +42,13 @@ def test_the_rule_finds_a_load_in_flight():
     assert unwaited_loads(late)
     assert not unwaited_loads(late.replace("sc1", "sc1\\n\\ts_waitcnt vmcnt(0)"))
     assert not unwaited_loads('asm("global_load_lds_dwordx4 %0, off" :: "v"(p));')
+
+
+def test_the_build_refuses_spills_of_every_kernel_but_the_cross_check():
+    """The VALU decode (kivi_decode.hip) is a cross-check whose speed is not followed."""
+    kernels = set()
+    for path in SOURCES:
+        if os.path.basename(path) != "kivi_decode.hip":
+            kernels |= set(re.findall(r"__global__[^;{]*?void\s+(?:__attribute__\S+\s+)?(\w+)\s*\(",
+                                      open(path).read()))
+    assert len(kernels) >= 3 and kernels == set(build.NO_SCRATCH)
