@@ -2279,28 +2279,28 @@ static void launch_one(const KiviGeo& g, const DecodeArgs& a, hipStream_t stream
 }
 
 // To the chunk kernel go all calls of the v1 symbols, whose queries must decode
-// to the same bits alone and together, and of the others those that no mix of lengths
-// makes slower here than in the stream.  The host knows the S segments and a bound U on
+// to the same bits alone and together, and of the others those that gain more here than
+// a bad mix of lengths loses.  The host knows the S segments and a bound U on
 // a segment's units (from the block table's width), not the lengths.  Where W workgroups
 // are resident, a long segment is sure of C = W / S of them, and with just over
 // (W - S) / C long segments among short ones it gets no more while S / W of the chip
 // idles: the longest run is then longer than the stream's equal ones by U / C units per
 // workgroup, times S / W.  What the chunk kernel saves is the stream's merge, a fixed
 // time.  So the bound is on S U / C per resident wavefront (`share`).  Stream / chunk in us
-// where the two meet, for the worst mix found:
-//  - HD 128, G <= 8, 12 units: 17 sequences (8 kv heads), 16 of them of 8352 tokens, 55.6 /
-//    57.3; 32, one of 4288, 35.1 / 35.3.  Equal lengths: 17 of 4000 tokens 42.7 / 34.3,
-//    of 16000 (beyond the bound) 84.0 / 102.7.  In workgroups of four
-//    wavefronts 5: 72 sequences, 25 of 352 tokens (4 units), 24.8 / 22.7, 25 of 704 (6
-//    units) 26.5 / 28.7.
-//  - HD 128, G > 8, whose stream folds one partial a round, 18: 44 sequences (2 kv
-//    heads), 43 of 26464 tokens, 107.1 / 98.5, of 35424 (24 units) 124.0 / 125.9.  In
-//    workgroups of four wavefronts 15: 132, 125 of 3392 tokens, 58.2 / 57.0, of 4128
-//    (18 units) 62.6 / 65.8.
-//  - HD 64, whose stream folds eight partials a round, 5: 44 (2 kv heads), 43 of 13056
-//    tokens (6 units), 41.8 / 40.6, of 17536 (8 units) 47.6 / 50.3; 3 where no segment is
-//    sure of a cut (C = 1): 96, 33 of 1216 tokens, 18.5 / 17.9, of 1728 (4 units) 19.3 /
-//    19.9; in workgroups of four wavefronts none that may be cut (132 of 300 tokens 17.5 / 18.0).
+// at the bound, for equal lengths and for the worst mix found:
+//  - HD 128, G <= 8: 12 units; 32 sequences (8 kv heads) of 4288 tokens 51.8 / 42.0, one of
+//    them among short ones 28.6 / 35.0.  10 where equal lengths leave more than 3 / 10 of the
+//    workgroups idle: 17 of 4000 tokens (6 units) 39.5 / 35.0, 16 of them 38.6 / 34.4, but of
+//    8352 (12 units) 56.8 / 58.9 and 54.3 / 57.0.  4 in workgroups of four wavefronts: 72 of
+//    352 tokens 28.4 / 23.8, 25 of them 23.1 / 22.7, of 512 (5 units) 34.6 / 28.3 and
+//    23.2 / 26.8.
+//  - HD 128, G > 8, whose stream folds one partial a round: 18; 44 sequences (2 kv heads) of
+//    26464 tokens 111.4 / 103.4, 43 of them 98.0 / 94.0.  In workgroups of four wavefronts 15:
+//    132 of 3392 tokens 64.3 / 58.7, 125 of them 54.6 / 56.8.
+//  - HD 64, whose stream folds eight partials a round: 5; 44 sequences (2 kv heads) of
+//    10848 tokens 36.3 / 36.8, 43 of them 35.6 / 36.0.  3 where no segment is sure of a cut
+//    (C = 1): 96 of 1216 tokens 20.9 / 19.1, 33 of them 17.1 / 17.9.  In workgroups of four
+//    wavefronts no segment that may be cut.
 // A call under a wide table may so take the stream where the same lengths under a tight
 // one come here.
 // How they are cut:
@@ -2332,8 +2332,9 @@ ChunkPlan plan_chunks(const KiviGeo& g, int batch, int64_t max_tokens, bool per_
   if (!per_query) {
     if (segs > slots || batch > 64 * kChunkWindows) return p;
     const int64_t cuts = slots / segs;
-    const int64_t share = segs > cus ? (g.hd == 64 ? 0 : wide ? 15 : 5)
-                                     : (g.hd == 64 ? (cuts > 1 ? 5 : 3) : wide ? 18 : 12);
+    const int64_t full = 10 * segs * cuts < 7 * slots ? 10 : 12;
+    const int64_t share = segs > cus ? (g.hd == 64 ? 0 : wide ? 15 : 4)
+                                     : (g.hd == 64 ? (cuts > 1 ? 5 : 3) : wide ? 18 : full);
     if (units > whole && segs * units > share * cuts * most * cus) return p;
   }
   p.waves = waves;

@@ -22,12 +22,13 @@ def plan(nh, nkv, hd, page, R, batch, tokens, per_query=0, cus=CUS):
     return dict(zip(("waves", "grid", "slots", "units", "whole"), out))
 
 
-# (heads, batch, longest): 5 to 36% slower in the chunk kernel for the lengths named
+# (heads, batch, longest): 3 to 36% slower in the chunk kernel for the lengths named
 @pytest.mark.parametrize("nh,nkv,hd,page,batch,tokens", [
     (40, 8, 128, 16, 17, 16000),  # equal lengths: one workgroup on 136 of 256 CUs
+    (40, 8, 128, 16, 17, 8400), (40, 8, 128, 16, 11, 30000),  # equal
     (40, 8, 128, 16, 11, 40000),  # equal: two on 88
     (40, 8, 128, 16, 20, 14000),  # 13 long ones among 7 short
-    (40, 8, 128, 16, 72, 1376),   # 25 long ones
+    (40, 8, 128, 16, 72, 1376), (40, 8, 128, 16, 72, 512),   # 25 long ones
     (40, 8, 128, 16, 96, 2752),   # a single long one
     (32, 2, 128, 32, 132, 5632),  # 125 long ones
     (14, 2, 64, 16, 44, 32000), (14, 2, 64, 16, 132, 4000), (14, 2, 64, 16, 192, 300),
