@@ -1914,8 +1914,13 @@ __device__ inline int chunk_units(const KiviGeo& g, const DecodeArgs& a,
     return wave_sum_i(c) * g.nkv <= slots;
   };
   int tot = 0;
+  bool cut = false;
 #pragma unroll
-  for (int w = 0; w < kChunkWindows; ++w) tot += units[w];
+  for (int w = 0; w < kChunkWindows; ++w) {
+    tot += units[w];
+    cut = cut || units[w] > a.chunk_whole;
+  }
+  if (!__builtin_amdgcn_ballot_w64(cut)) return a.chunk_units;  // every segment whole
   tot = wave_sum_i(tot) * g.nkv;
   int lo = max(a.chunk_units, (tot + slots - 1) / slots);
   if (fits(lo)) return lo;
@@ -2011,9 +2016,15 @@ __global__ __launch_bounds__(64 * (coop_max_waves<HD, PACK>())) void kivi_decode
       before += __builtin_amdgcn_readlane(incl, 63);
     }
     if (b < 0) break;
-    const int h = rel / cnt, ci = rel - h * cnt;
+    int h = rel, ci = 0, u0 = 0, u1 = U;
+    if (cnt > 1) {
+      // 32 bits: a table addresses at most 2^18 tokens, so U, and cnt <= U, are below 2^15
+      h = (uint32_t)rel / (uint32_t)cnt;
+      ci = rel - h * cnt;
+      u0 = (uint32_t)(ci * U) / (uint32_t)cnt;
+      u1 = (uint32_t)((ci + 1) * U) / (uint32_t)cnt;
+    }
     const int nq = ov / kGroup;
-    int u0 = (int)((int64_t)ci * U / cnt), u1 = (int)((int64_t)(ci + 1) * U / cnt);
 
     // ---- fused step: the last chunk writes ----
     int g_age = 0x7fffffff, new_row = -1, Lb = 0;
@@ -2045,14 +2056,20 @@ __global__ __launch_bounds__(64 * (coop_max_waves<HD, PACK>())) void kivi_decode
     }
 
     // ---- this wavefront's run of the chunk ----
-    const int ua = u0 + (int)((int64_t)(u1 - u0) * wv / nw),
-              ub = u0 + (int)((int64_t)(u1 - u0) * (wv + 1) / nw);
+    auto share = [&](int w) {  // units before wavefront w's; nw is 4, 8 or 12
+      const uint32_t x = (uint32_t)((u1 - u0) * w);
+      return u0 + (int)(nw == 12 ? x / 12 : nw == 8 ? x / 8 : x / 4);
+    };
+    const int ua = share(wv), ub = share(wv + 1);
     const int t_beg = tile_at(ua, nq), t_fin = tile_at(ub, nq);
     // the ones block of every stage (the DMAs never write it; a partial may have)
     if (lane < 32) {
 #pragma unroll
       for (int s_ = 0; s_ < S; ++s_) ((uint32_t*)ring[s_].ones)[lane] = 0x3C003C00u;
     }
+    // one tile in all (sequences of up to 32 tokens): its wavefront writes O from its
+    // registers, 0.4 us less than by way of LDS
+    const bool single = cnt == 1 && nq + (n - ov + kGroup - 1) / kGroup <= 1;
     WaveState<HD> st;
     float* ml = (float*)mine;       // partial: (m, l) per head, 16 of them, then acc
     float* acc = (float*)mine + 32;
@@ -2081,29 +2098,46 @@ __global__ __launch_bounds__(64 * (coop_max_waves<HD, PACK>())) void kivi_decode
       decode_tiles<HD, P, PACK, FUSED>(g, a, ring, qrows, nb, sscale, lane, b, h, ov, n, t_beg,
                                        t_fin, g_age, new_row, ages, st, no_wait, progress,
                                        t_first);
-      // ---- its partial to LDS (the ring is idle: every DMA has landed) ----
       int ln = lane;
       asm volatile("" : "+v"(ln));
       const int c = ln & 15, j = ln >> 4;
       const bool sum_col = sum_lane<HD>(c);
+      if (single) {  // O from its registers
+        float* const out = a.out + (int64_t)b * a.out_stride + (int64_t)h * G * HD;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float left = __shfl(st.ob[i], ln - 1, 64);
-        const float z = sum_col ? left : st.ob[i];
-        if (4 * j + i < G) {
-          float* p = acc + (4 * j + i) * HD + CPL * c;
+        for (int i = 0; i < 4; ++i) {
+          const float left = __shfl(st.ob[i], ln - 1, 64);
+          const float z = sum_col ? left : st.ob[i];
+          const float inv = 1.0f / fmaxf(__shfl(st.ob[i], 16 * j + C1, 64), 1.0e-30f);
+          if (4 * j + i < G) {
+            float* p = out + (4 * j + i) * HD + CPL * c;
 #pragma unroll
-          for (int q4 = 0; q4 < CPL / 4; ++q4)
-            *(floatx4*)(p + 4 * q4) = floatx4{st.o[4 * q4][i] + z, st.o[4 * q4 + 1][i] + z,
-                                              st.o[4 * q4 + 2][i] + z, st.o[4 * q4 + 3][i] + z};
-          if (c == C1) ml[2 * (4 * j + i) + 1] = st.ob[i];  // Sigma P of head 4j + i
+            for (int q4 = 0; q4 < CPL / 4; ++q4)
+              *(floatx4*)(p + 4 * q4) =
+                  floatx4{st.o[4 * q4][i] + z, st.o[4 * q4 + 1][i] + z, st.o[4 * q4 + 2][i] + z,
+                          st.o[4 * q4 + 3][i] + z} * inv;
+          }
         }
+      } else {  // its partial to LDS (the ring is idle: every DMA has landed)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float left = __shfl(st.ob[i], ln - 1, 64);
+          const float z = sum_col ? left : st.ob[i];
+          if (4 * j + i < G) {
+            float* p = acc + (4 * j + i) * HD + CPL * c;
+#pragma unroll
+            for (int q4 = 0; q4 < CPL / 4; ++q4)
+              *(floatx4*)(p + 4 * q4) = floatx4{st.o[4 * q4][i] + z, st.o[4 * q4 + 1][i] + z,
+                                                st.o[4 * q4 + 2][i] + z, st.o[4 * q4 + 3][i] + z};
+            if (c == C1) ml[2 * (4 * j + i) + 1] = st.ob[i];  // Sigma P of head 4j + i
+          }
+        }
+        if (j == 0 && c < G) ml[2 * c] = st.m;
       }
-      if (j == 0 && c < G) ml[2 * c] = st.m;
     } else if (lane < G) {
       ml[2 * lane] = -INFINITY;  // no tile: skipped below
     }
-    __syncthreads();
+    if (!single) __syncthreads();
 
     // ---- the chunk: fold the wavefronts' partials in order ----
     // an opaque thread id: addresses formed from here on are not computed (and
@@ -2125,7 +2159,7 @@ __global__ __launch_bounds__(64 * (coop_max_waves<HD, PACK>())) void kivi_decode
             *(const u32x4*)nx;
       }
     }
-    const int n4 = G * HD / 4;
+    const int n4 = single ? 0 : G * HD / 4;
     const bool whole = cnt == 1;
     float* const out = a.out + (int64_t)b * a.out_stride + (int64_t)h * G * HD;
     for (int e = tid; e < n4; e += blockDim.x) {

@@ -105,3 +105,31 @@ def test_v1_queries_of_two_launches_equal_single():
     for i in list(range(0, 160, 13)) + [1, 2, 3, 88, 89, 90, 159]:
         kivi.kivi_decode_dsl(q[i].contiguous(), bt, *pool, int(seq[i]), one)
         assert torch.equal(one.view(torch.int32), out[i].view(torch.int32)), i
+
+
+@pytest.mark.parametrize("nh,nkv,hd,page", [(10, 2, 128, 16), (32, 2, 128, 32), (14, 2, 64, 16),
+                                            (20, 2, 64, 32)])
+def test_one_tile_sequences_equal_the_stream(nh, nkv, hd, page):
+    """A sequence of up to 32 tokens is one wavefront's, which writes O from its registers in
+    both kernels: the same bits, beside longer sequences and with none."""
+    from jacq_amd import kivi
+    for lens in ([0, 1, 31, 32], [32, 33, 200, 7, 1000]):
+        w = wl.Workload("short", nh, nkv, hd, len(lens), 1, 1, page=page, residual=64, outliers=2,
+                        outlier_scale=9.0, seed=5)
+        st = State(w, lens=lens, seed=hd)
+        st.build_oracle()
+        geo = kivi.KiviGeometry(nh, nkv, hd, page, 32, 64, st.max_pages, st.num_pages)
+        cache = kivi.PagedKiviCache.from_tensors(geo, to_torch(st))
+        q = torch.from_numpy(st.q).view(torch.float16).cuda()
+        args = (q, torch.from_numpy(st.lens.astype(np.int32)).cuda(),
+                torch.from_numpy(st.tables).cuda())
+        chunk = cache.decode(*args)
+        kivi.lib().jacq_kivi_test_force_stream(1)
+        try:
+            stream = cache.decode(*args)
+        finally:
+            kivi.lib().jacq_kivi_test_force_stream(0)
+        assert_close(chunk.cpu().numpy(), st.decode_ref(), "decode")
+        for b, n in enumerate(lens):
+            if n <= 32:
+                assert torch.equal(chunk[b].view(torch.int32), stream[b].view(torch.int32)), n
