@@ -64,7 +64,7 @@ __global__ __launch_bounds__(64 * (HD / kGroup)) void kivi_append_kernel(KiviGeo
   if (x < 2 * g.nkv) {
     const AppendSpan sp(g, start, a.num_new);
     if (__builtin_expect(sp.D == 0, 1))  // first, and short: most calls fetch no other code
-      append_rows<HD, false>(g, a, b, x >> 1, x & 1, wave, sp.r0, a.num_new, lane);
+      append_rows<HD>(g, a, b, x >> 1, x & 1, wave, sp.r0, a.num_new, lane);
     else if (x & 1)
       append_slice<HD, true, false>(g, a, b, x >> 1, wave, start, a.num_new, lane, [] {});
     else
