@@ -152,6 +152,7 @@ def main() -> int:
                    kivi.lib().jacq_kivi_write_decode_workspace_size(ctypes_geo(kivi, geo), B))
     workspace = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
 
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
     stream = torch.cuda.current_stream(dev)
     STAMP_CAP = 8192  # workgroups per launch the stamp buffer holds
     stamps = (torch.zeros((args.steps, STAMP_CAP, 4), dtype=torch.int64, device=dev)
@@ -319,8 +320,8 @@ def main() -> int:
         "hbm_frac": round(gbs / HBM_PEAK_GBS, 4),
         "wall_s_timed_region": round(wall, 4),
         "roofline": {
-            "kernel": f"kivi_decode_stream_kernel<{w.hd}, {w.page}, "
-                      f"{'true' if w.nh // w.nkv <= 8 else 'false'}, false, true> "
+            "kernel": f"kivi_decode_{decode_kernel(kivi, geo, B, cus)}_kernel<{w.hd}, {w.page}, "
+                      f"{'true' if w.nh // w.nkv <= 8 else 'false'}, true> "
                       f"(fused write + decode)",
             "bound": "hbm",
             "achieved": round(gbs, 1),
@@ -355,6 +356,15 @@ def copy_calibration(torch, dev, mib: int) -> int:
 def ctypes_geo(kivi, geo):
     import ctypes
     return ctypes.byref(geo.c())
+
+
+def decode_kernel(kivi, geo, batch, cus):
+    """Which matrix-core kernel a call of this batch and table takes on `cus` CUs."""
+    import ctypes
+    plan = (ctypes.c_int32 * 5)()
+    kivi.lib().jacq_kivi_test_plan_decode(ctypes_geo(kivi, geo), batch,
+                                          ctypes.c_int64(geo.max_seq_len()), 0, cus, plan)
+    return "chunk" if plan[0] else "stream"
 
 
 def load_traffic(workload: str):

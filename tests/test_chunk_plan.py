@@ -85,3 +85,12 @@ def test_every_chunk_has_a_workgroup_and_a_workspace_slot():
         n = device_chunks([units(x) for x in lens], nkv, p)
         assert n <= p["grid"] <= max(p["slots"], batch * nkv)
     assert taken > 500
+
+
+def test_bench_names_the_kernel_that_runs():
+    import bench
+    for (nh, nkv, hd, batch, pages), want in (((40, 8, 128, 64, 1024), "stream"),
+                                              ((32, 8, 128, 32, 256), "chunk"),
+                                              ((32, 4, 64, 1, 40), "chunk")):
+        geo = kivi.KiviGeometry(nh, nkv, hd, 16, 32, 128, pages, 1 << 16)
+        assert bench.decode_kernel(kivi, geo, batch, CUS) == want
