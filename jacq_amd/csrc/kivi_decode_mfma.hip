@@ -327,15 +327,15 @@ __device__ inline void wait_stages(int later) {
     wait_vm<0>();
 }
 
-// LDS stages per wave: S - 1 groups in flight while one is computed.
 // LDS stages and waves per SIMD of each kernel.  Two waves per SIMD do not
 // hide one wave's dependency chain (LDS read, unpack, QK MFMA chain, max, exp,
 // PV), so the packed HD=128 kernel (G <= 8, the common GQA shapes) runs three
 // per SIMD: at most 168 VGPRs, and two 5 KiB stages per wave so that 12 waves'
 // rings fit the CU's 160 KiB of LDS (one group in flight while one is
 // computed: the memory latency is below a group's compute time).  The other
-// kernels keep three stages; their register use already allows three waves
-// (HD=64) or would spill at three (HD=128, G > 8).
+// kernels keep three stages (two groups in flight): at HD=64 twelve waves fit
+// with them, at HD=128 and G > 8 (16 Q rows too) eight do, and eleven with two stages
+// were no faster.
 template <int HD, bool PACK>
 constexpr int stages() {
   return (HD == 128 && PACK) ? 2 : 3;

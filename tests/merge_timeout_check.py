@@ -1,8 +1,8 @@
 """Child process of test_gpu_parity.test_merge_timeout_exits_v1_symbols.
 
-With the library's test hook every merge wait of a decode runs out.  The
-first jac_launch (v1 geometry, one 4096-token sequence, whose split-K pieces
-need merging) returns and drains; the second sees the device's time-out
+With the library's test hook a decode's fold across workgroups fails as if its
+wait had run out.  The first jac_launch (v1 geometry, one 4096-token sequence,
+whose chunks need folding) returns and drains; the second sees the device's time-out
 status and must print the error and exit(1), as the v1 symbols do for launch
 errors.  Prints FIRST_DECODE_RETURNED between the two calls."""
 from __future__ import annotations

@@ -130,8 +130,9 @@ def _go_on(st, starts, ends):
 
 
 def test_code_by_reciprocal_equals_division():
-    """The writer takes rint((x - min) * rcp(scale)) where that lies further
-    than 2^-16 from a rounding boundary and divides elsewhere: with any
+    """The rule that the writer's codes follow (the kernel's own are in
+    test_codes_at_half_codes): rint((x - min) * rcp(scale)) where that lies further
+    than 2^-16 from a rounding boundary, a division elsewhere.  With any
     reciprocal within 1 ulp, every code it takes is the division's, over fp16
     tiles of every exponent and quotients placed at the boundaries."""
     rng = np.random.default_rng(7)

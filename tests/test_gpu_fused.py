@@ -96,8 +96,8 @@ def test_write_decode_every_sequence_ages_out(kivi, name):
 def test_write_decode_equals_append_then_decode(kivi):
     """The fused step leaves the same cache bits as jacq_kivi_cache_append
     followed by jacq_kivi_decode, and decodes to the same values within the
-    rounding of its own run split (its writer wavefronts take shorter runs,
-    so the decode's cut differs)."""
+    rounding of its own split (the last chunk takes all of what it writes; in the
+    stream, test_gpu_stream.py, writer wavefronts take shorter runs)."""
     w = wl.WORKLOADS["qwen14b"].scaled(batch=8, ctx_lo=1000)
     lens = np.array([1000, 2207, 4095, 159, 160, 3000, 5000, 2048])
     st = State(w, lens=lens, extra_tokens=1, seed=53)
@@ -129,9 +129,10 @@ def test_write_decode_equals_append_then_decode(kivi):
 
 
 def test_write_decode_graph_replays(kivi):
-    """The fused step captured in a HIP graph (the writer flags are cleared by
-    the wavefront or merge that finishes each aging segment, so a replay,
-    which repeats the launch's epoch, starts from zero flags): replays with new
+    """The fused step captured in a HIP graph (flags are cleared by whoever
+    finishes a segment -- the chunks' flags here, the stream's writer flags too in
+    test_gpu_stream.py -- so a replay, which repeats the launch's epoch, starts
+    from zero flags): replays with new
     tokens and lengths copied in between advance the cache exactly as eager
     fused steps do, bit for bit, across age-outs."""
     w = wl.WORKLOADS["qwen14b"].scaled(batch=4, ctx_lo=150)
@@ -204,8 +205,9 @@ def test_write_decode_other_geometries(kivi, name):
 
 
 def test_write_decode_merge_timeout_is_reported(kivi):
-    """Failure handling in the fused step, forced from the host (the merge
-    waits for a tag nobody stores and gives up after 20 us): the launch ends,
+    """Failure handling in the fused step, forced from the host (the stream's
+    merge waits for a tag nobody stores and gives up after 20 us, test_gpu_stream.py;
+    the chunk kernel poisons what it folds): the launch ends,
     the writer's work is complete and bit-exact (it waits for nothing), whole
     segments decode correctly and merged ones are NaN; the next fused step is
     refused without launching (cache and output untouched) until

@@ -223,9 +223,8 @@ def test_v1_jac_launch_all_boundaries(kivi):
 def test_v1_batched_decode_equals_single(kivi):
     """jac_launch_batched equals jac_launch per query bit for bit
     (variants.rs:1211-1213): the v1 symbols cut each query's work by its own
-    length alone.  60 causal queries up to the 4096-token v1 maximum need
-    more than one launch of the static workspace region, which must not
-    change any query's bits either."""
+    length alone.  60 causal queries up to the 4096-token v1 maximum take one
+    launch (160 take two: test_v1_queries_of_two_launches_equal_single)."""
     st = State(V1, lens=[4096], seed=8)
     st.build_oracle()
     g = to_torch(st)
@@ -666,9 +665,10 @@ def _segment_counts(w, got, ref):
 
 
 def test_merge_timeout_drains_and_is_reported(kivi):
-    """Failure handling of the in-launch merge, forced from the host: with the
-    test hook the merge waits for a tag nobody stores and gives up after
-    20 us.  The launch still ends; segments a single wavefront wrote whole stay
+    """Failure handling of the fold across workgroups, forced from the host:
+    with the test hook the stream's merge waits for a tag nobody stores and gives
+    up after 20 us (test_gpu_stream.py); the chunk kernel, which such a call takes
+    by itself and which waits for nothing, poisons what it folds.  The launch still ends; segments a single wavefront wrote whole stay
     correct and every merged segment is NaN.  The device's status word is set:
     the next decode is refused (nothing launched), jacq_kivi_decode_status
     reports the time-out once and resets, and decodes are correct again."""
@@ -707,8 +707,9 @@ def test_merge_timeout_drains_and_is_reported(kivi):
 def test_merge_timeout_poisons_graph_replays(kivi):
     """A graph replay never passes through the host's status check, and it
     repeats its launch epoch: after a merge on its workspace timed out, flags
-    that the late stream wavefronts stored would look like the replay's own.
-    The timed-out merge poisons the workspace, so the replays' merged segments
+    that late stream wavefronts stored would look like the replay's own (the
+    stream runs in test_gpu_stream.py; the chunk kernel has the same contract).
+    What timed out poisons the workspace, so the replays' merged segments
     are NaN -- never finite values built from stale partials -- until
     jacq_kivi_decode_status zeroes the workspace; then replays equal the
     eager decode again."""
@@ -772,9 +773,9 @@ def test_merge_timeout_exits_v1_symbols(kivi):
 
 
 def test_wave_stamps_cover_the_stream(kivi):
-    """The profiling hook (jacq_kivi_profile_wave_stamps): every stream
-    workgroup stamps an end after its start, and their units add up to the
-    stream's total (sum over sequences and kv heads of quantised groups plus
+    """The profiling hook (jacq_kivi_profile_wave_stamps): every workgroup (of
+    the chunk kernel here, of the stream in test_gpu_stream.py) stamps an end
+    after its start, and their units add up to the call's total (sum over sequences and kv heads of quantised groups plus
     three units per fp16 residual tile)."""
     from jacq_amd import cache_io
     w = wl.WORKLOADS["qwen14b"].scaled(batch=4, ctx_lo=900)
